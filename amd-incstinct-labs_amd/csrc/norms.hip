@@ -1,5 +1,6 @@
 // Runtime norm and RoPE entry points for gfx950: RMSNorm, two-pass LayerNorm and row softmax with
-// one wave per row (DPP/permlane butterfly reductions, zero LDS), rotate-half RoPE with one
+// one wave per row (DPP/permlane butterfly reductions, zero LDS; wide, unaligned and few rows go to
+// rows_wide.hip), rotate-half RoPE with one
 // thread per (d, d + D/2) pair, and the RoPE cos/sin table built on the device.
 //
 // Reference behaviour restated:
@@ -9,6 +10,7 @@
 //   rope_kernel         cdna3-prims/include/cdna3/runtime/forward.hpp:135-148
 //   Session::fill_rope  cdna3-prims/include/cdna3/runtime/session.hpp:120-135
 #include "common.hpp"
+#include "rows_wide.hpp"
 #include "wave_primitives/detail/xlane.hpp"
 
 namespace cdna4 {
@@ -123,7 +125,8 @@ __global__ __launch_bounds__(256) void rmsnorm_row16(const float* __restrict__ X
     }
 }
 
-// Any H and alignment: two passes over the row (the second pass hits the cache).
+// Rows of fewer than 4 or more than 65,536 columns that the other forms do not take: two passes over
+// the row (the second pass hits the cache).
 __global__ __launch_bounds__(256) void rmsnorm_any(const float* __restrict__ X, const uint16_t* __restrict__ W,
                                                    float* __restrict__ Y, int M, int H, float eps) {
     const unsigned lane = threadIdx.x & 63u;
@@ -236,7 +239,7 @@ __global__ __launch_bounds__(256) void layernorm_any(const float* __restrict__ X
 // The reference's order of work: the row maximum (DPP max), exp(x - m) (__expf), their sum (DPP
 // sum), then each value times 1 / sum. Columns past H take -inf into the maximum and 0 into the
 // sum. Same row layouts as the norms: one wave per row with the row in registers (H <= 256 NV),
-// 16 lanes per row for H <= 64, two passes for anything else.
+// 16 lanes per row for H <= 64; wide, unaligned and few rows go to rows_wide.hip.
 template <int NV, bool kNT>
 __global__ __launch_bounds__(256) void softmax_vec(const float* __restrict__ X, float* __restrict__ Y, int M, int H) {
     const unsigned lane = threadIdx.x & 63u;
@@ -368,11 +371,12 @@ extern "C" int cdna3_rmsnorm_f32(const float* X, const void* W, float* Y, int M,
     const unsigned grid = ceil_div((size_t)M, kNormWaves);
     const uint16_t* w = (const uint16_t*)W;
     const bool vec = (H % 4 == 0) && H <= 4096 && aligned16(X) && aligned16(Y) && (((uintptr_t)W & 7u) == 0);
+    const bool nt = (size_t)M * (size_t)H * sizeof(float) >= kStreamBytes;
+    if (rows_wide_takes(M, H, vec)) return rows_wide(kRowsRms, X, W, nullptr, Y, M, H, eps, nt, s);
     if (!vec) {
         rmsnorm_any<<<grid, 256, 0, s>>>(X, w, Y, M, H, eps);
         return launch_status();
     }
-    const bool nt = (size_t)M * (size_t)H * sizeof(float) >= kStreamBytes;
     if (H <= 64) {
         if (nt) rmsnorm_row16<true><<<ceil_div((size_t)M, kRows16 * kRowsPerLane), 256, 0, s>>>(X, w, Y, M, H, eps);
         else rmsnorm_row16<false><<<ceil_div((size_t)M, kRows16 * kRowsPerLane), 256, 0, s>>>(X, w, Y, M, H, eps);
@@ -393,11 +397,12 @@ extern "C" int cdna3_layernorm_f32(const float* X, const float* gamma, const flo
     hipStream_t s = (hipStream_t)stream;
     const unsigned grid = ceil_div((size_t)M, kNormWaves);
     const bool vec = (H % 4 == 0) && H <= 4096 && aligned16(X) && aligned16(Y) && aligned16(gamma) && aligned16(beta);
+    const bool nt = (size_t)M * (size_t)H * sizeof(float) >= kStreamBytes;
+    if (rows_wide_takes(M, H, vec)) return rows_wide(kRowsLayer, X, gamma, beta, Y, M, H, eps, nt, s);
     if (!vec) {
         layernorm_any<<<grid, 256, 0, s>>>(X, gamma, beta, Y, M, H, eps);
         return launch_status();
     }
-    const bool nt = (size_t)M * (size_t)H * sizeof(float) >= kStreamBytes;
     if (H <= 64) {
         if (nt) layernorm_row16<true><<<ceil_div((size_t)M, kRows16 * kRowsPerLane), 256, 0, s>>>(X, gamma, beta, Y, M, H, eps);
         else layernorm_row16<false><<<ceil_div((size_t)M, kRows16 * kRowsPerLane), 256, 0, s>>>(X, gamma, beta, Y, M, H, eps);
@@ -417,11 +422,12 @@ extern "C" int cdna3_softmax_rows_f32(const float* X, float* Y, int M, int H, cd
     hipStream_t s = (hipStream_t)stream;
     const unsigned grid = ceil_div((size_t)M, kNormWaves);
     const bool vec = (H % 4 == 0) && H <= 4096 && aligned16(X) && aligned16(Y);
+    const bool nt = (size_t)M * (size_t)H * sizeof(float) >= kStreamBytes;
+    if (rows_wide_takes(M, H, vec)) return rows_wide(kRowsSoftmax, X, nullptr, nullptr, Y, M, H, 0.f, nt, s);
     if (!vec) {
         softmax_any<<<grid, 256, 0, s>>>(X, Y, M, H);
         return launch_status();
     }
-    const bool nt = (size_t)M * (size_t)H * sizeof(float) >= kStreamBytes;
     if (H <= 64) {
         if (nt) softmax_row16<true><<<ceil_div((size_t)M, kRows16 * kRowsPerLane), 256, 0, s>>>(X, Y, M, H);
         else softmax_row16<false><<<ceil_div((size_t)M, kRows16 * kRowsPerLane), 256, 0, s>>>(X, Y, M, H);
