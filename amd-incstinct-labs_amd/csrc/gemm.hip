@@ -22,7 +22,7 @@
 // of one read then touch every bank once, and a lane's four accumulator values are four
 // consecutive output columns n (one 16-byte or 8-byte store). Wave (wm, wn) takes block u = wn of
 // every W group and u = wm of every X group of the tile. Rows past M or N read the last valid row
-// (their results are not stored).
+// (their results are not stored). Large products take 256-row tiles of eight waves (gemm_big, below).
 #include "attn_stream.hpp"
 
 namespace cdna4 {
@@ -262,6 +262,185 @@ __global__ __launch_bounds__(256) void gemm_ring(const uint16_t* __restrict__ X,
     }
 }
 
+// ---- large products: 256 x 256 and 256 x 128 tiles, eight waves ------------------------------
+// One workgroup per CU, two waves per SIMD, wave (wm, wn) of WM x 8 / WM: 128 X rows x 64 W rows of
+// a 256 x 256 tile (12 operand reads per 32 MFMAs), 64 x 64 of a 256 x 128 one (8 per 16). A stage
+// (64-wide K of both operand tiles, the LDS layout above) is two K steps; the operands of a step are
+// read during the MFMAs of the step before it, so the matrix cores wait for LDS only at the start:
+//   step 0 of stage t: MFMAs; reads of stage t, step 1
+//   wait for the copies of stage t + 1; barrier: stage t + 1 is visible, and stage t is in registers
+//   step 1 of stage t: MFMAs; reads of stage t + 1, step 0; copies of stage t + 2 into stage t's slot
+// Two slots (128 KB) then keep the copies behind the MFMAs with one barrier per stage.
+// What bounds it is the matrix cores at the clock the board's power limit leaves them (random fp16
+// operands), then the barrier. Measured, f16 unless said (us, before: 128 x 128 ring tiles): 4096^3
+// 185 -> 110 (1,250 TFLOP/s; rocBLAS 95-108), 8192^3 1,371 -> 815, SiLU 4096 x 8192 x 4096 734 -> 428,
+// 2048 x 4096 x 4096 (256 x 128) 87.6 -> 72, 2048 x 3072 x 1024 22.2 -> 19.5.
+// Tried and slower: 32-wide stages in a ring of four (a barrier per step; 119 against 112 at 4096^3),
+// four waves of 128 x 128 with the accumulators in AGPRs (127), 128 x 128 tiles of eight waves (217).
+// Level: three or four operand reads per slot, wave priority raised around the MFMAs.
+// Tile of workgroup b (XCD b % 8): each XCD takes a contiguous part of the tiles in an order that
+// runs through groups of 8 m tiles, m fastest, so the 32 workgroups of an XCD share 8 X and 4 W
+// tiles in its L2 at a time.
+__device__ __forceinline__ void big_tile_of(int b, int tm, int tn, int& mt, int& nt) {
+    const int total = tm * tn, q = total >> 3, r = total & 7, x = b & 7;
+    const int i = x * q + min(x, r) + (b >> 3);
+    constexpr int kGroup = 8;
+    const int grp = i / (kGroup * tn), m0 = grp * kGroup, gm = min(kGroup, tm - m0), in = i - grp * kGroup * tn;
+    mt = m0 + in % gm;
+    nt = in / gm;
+}
+
+template <int BM, int BN, int WM, int kOut, bool kAccum>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_big(
+    const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, void* __restrict__ Y, int M, int N, int K, int ldy) {
+    constexpr bool kSilu = kOut == kOutSilu;
+    static_assert(kOut != kOutQKV && !(kSilu && kAccum), "output forms");
+    constexpr int kTileCols = kSilu ? BN / 2 : BN;
+    constexpr int kStage = (BN + BM) * kRowBytes;
+    constexpr int WN = 8 / WM;                            // waves across W
+    constexpr int FM = BM / WM / 16, FN = BN / WN / 16;   // 16-row blocks per wave: X, W
+    constexpr int NCW = BN / 64, NC = (BN + BM) / 64;     // copies per wave and stage: of W, in all
+    static_assert(FM % 2 == 0 && FN % 2 == 0 && (!kSilu || FN == 4), "waves take whole 32-row groups");
+    const int ncols = kSilu ? N / 2 : N;
+    __shared__ __attribute__((aligned(16))) char lds[2 * kStage];
+
+    const int lane = (int)(threadIdx.x & 63u);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int li = lane & 15, g = lane >> 4;
+    const int wm = wave % WM, wn = wave / WM;
+    int mt, nt;
+    big_tile_of((int)blockIdx.x, (M + BM - 1) / BM, (ncols + kTileCols - 1) / kTileCols, mt, nt);
+    const int m0 = mt * BM, n0 = nt * kTileCols;
+
+    // Copy j of a wave is instruction c = wave + 8 j of a stage (rows 8 c .. 8 c + 7): W for j < NCW.
+    uint32_t coff[NC];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const int row = (wave + 8 * j) * 8 + (lane >> 3);
+        const int chunk = (lane & 7) ^ tile::swz_k<64>(row & 31);
+        int r;
+        if (j >= NCW) r = min(m0 + row - BN, M - 1);
+        else if (kSilu) r = row < BN / 2 ? min(n0 + row, ncols - 1) : ncols + min(n0 + row - BN / 2, ncols - 1);
+        else r = min(n0 + row, N - 1);
+        coff[j] = (uint32_t)r * (uint32_t)K * 2u + (uint32_t)chunk * 16u;
+    }
+    auto copy = [&](int kt, int j) {
+        stream::dma16_s((j < NCW ? W : X) + (size_t)kt * kBK, coff[j], lds + (kt & 1) * kStage + (wave + 8 * j) * 1024);
+    };
+
+    // Operand rows of the wave: FN / 2 W groups (32 rows, blocks u = 0, 1) and FM / 2 X groups, both
+    // consecutive; a SiLU tile's wave takes a gate group and the up group of the same columns.
+    const int r0 = 8 * (li >> 2) + (li & 3);
+    const uint32_t rd = (uint32_t)(r0 * kRowBytes + ((g ^ tile::swz_k<64>(r0)) * 16));
+    constexpr uint32_t kWStep = (kSilu ? WN : 1) * 4096u;   // bytes from one W group of the wave to the next
+    const uint32_t rw = rd + (uint32_t)(kSilu ? wn : FN / 2 * wn) * 4096u;
+    const uint32_t rx = rd + (uint32_t)(BN * kRowBytes) + (uint32_t)wm * (FM / 2) * 4096u;
+    struct Ops { u32x4 a[FN], b[FM]; };
+    auto read_a = [&](Ops& o, const char* st, uint32_t flip, int i) {
+        o.a[i] = *(const u32x4*)(st + (rw ^ flip) + (i >> 1) * kWStep + (i & 1) * 512);
+    };
+    auto read_b = [&](Ops& o, const char* st, uint32_t flip, int j) {
+        o.b[j] = *(const u32x4*)(st + (rx ^ flip) + (j >> 1) * 4096 + (j & 1) * 512);
+    };
+
+    gf32x4 acc[FN][FM];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) acc[i][j] = gf32x4{0.f, 0.f, 0.f, 0.f};
+
+    const int nk = K / kBK;   // >= 2 (big_takes)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) copy(0, j);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) copy(1, j);
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(NC) : "memory");
+    __syncthreads();
+    Ops o0, o1;
+#pragma unroll
+    for (int i = 0; i < FN; ++i) read_a(o0, lds, 0u, i);
+#pragma unroll
+    for (int j = 0; j < FM; ++j) read_b(o0, lds, 0u, j);
+
+    constexpr int kReads = FM == 8 ? 2 : 4;   // operand reads per slot: all in the first slots
+    // One K step: FM slots of FN MFMAs on operands o; ahead of them, in the first slots, the reads of
+    // the next step's operands (rd_next) from st at K step `flip`, and the copies of stage kc (cp).
+    auto step = [&](const Ops& o, Ops& nx, const char* st, uint32_t flip, bool rd_next, int kc, bool cp) {
+#pragma unroll
+        for (int j = 0; j < FM; ++j) {
+            if (rd_next) {
+#pragma unroll
+                for (int r = j * kReads; r < min((j + 1) * kReads, FN + FM); ++r)
+                    if (r < FN) read_a(nx, st, flip, r);
+                    else read_b(nx, st, flip, r - FN);
+            }
+            if (cp) {
+#pragma unroll
+                for (int c = j * NC / FM; c < (j + 1) * NC / FM; ++c) copy(kc, c);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < FN; ++i)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gf16x8, o.a[i]),
+                                                                   __builtin_bit_cast(gf16x8, o.b[j]), acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    int kt = 0;
+    for (; kt + 2 < nk; ++kt) {
+        step(o0, o1, lds + (kt & 1) * kStage, 64u, true, 0, false);
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        __syncthreads();
+        step(o1, o0, lds + ((kt + 1) & 1) * kStage, 0u, true, kt + 2, true);
+    }
+    // the last two stages: nothing left to copy
+    step(o0, o1, lds + (kt & 1) * kStage, 64u, true, 0, false);
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    __syncthreads();
+    ++kt;
+    step(o1, o0, lds + (kt & 1) * kStage, 0u, true, 0, false);
+    step(o0, o1, lds + (kt & 1) * kStage, 64u, true, 0, false);
+    step(o1, o0, lds, 0u, false, 0, false);
+
+    // acc[i][j] lane (li, g): W group i / 2, block u = i % 2, so columns 8 g + 4 u + e of the group: a
+    // lane's two blocks of a group are eight consecutive columns of row m of X block j. (The lane's
+    // index is formed again: kept from the start it would take registers the loop has not.)
+    const int el = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const int er0 = 8 * ((el & 15) >> 2) + (el & 3), eg = el >> 4;
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+        const int m = m0 + 16 * FM * wm + 32 * (j >> 1) + er0 + 4 * (j & 1);
+        if (m >= M) continue;
+#pragma unroll
+        for (int h = 0; h < (kSilu ? 1 : FN / 2); ++h) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int n = n0 + (kSilu ? 32 * wn : 16 * FN * wn + 32 * h) + 8 * eg + 4 * u;
+                if (n >= ncols) continue;
+                gf32x4 v = acc[2 * h + u][j];
+                if constexpr (kSilu) {
+                    const gf32x4 up = acc[(2 + u) % FN][j];
+                    uint32_t q[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) q[e] = f32_to_f16_bits(v[e] / (1.f + expf(-v[e])) * up[e]);
+                    *(u32x2*)((uint16_t*)Y + (size_t)m * ldy + n) = u32x2{q[0] | (q[1] << 16), q[2] | (q[3] << 16)};
+                } else if constexpr (kOut == kOutF32) {
+                    float* y = (float*)Y + (size_t)m * ldy + n;
+                    if constexpr (kAccum) v += *(const gf32x4*)y;
+                    *(gf32x4*)y = v;
+                } else {
+                    _Float16* y = (_Float16*)Y + (size_t)m * ldy + n;
+                    if constexpr (kAccum) {
+                        const gf16x4 p = *(const gf16x4*)y;
+                        v += gf32x4{(float)p[0], (float)p[1], (float)p[2], (float)p[3]};
+                    }
+                    *(gf16x4*)y = gf16x4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+                }
+            }
+        }
+    }
+}
+
 template <int BM, int BN>
 int gemm_launch(const uint16_t* X, const uint16_t* W, void* Y, bool y_f32, bool accum, int M, int N, int K, int ldy,
                 hipStream_t s) {
@@ -273,6 +452,27 @@ int gemm_launch(const uint16_t* X, const uint16_t* W, void* Y, bool y_f32, bool 
         if (accum) gemm_ring<BM, BN, kOutF16, true><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldy, QkvOut{});
         else gemm_ring<BM, BN, kOutF16, false><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldy, QkvOut{});
     }
+    return launch_status();
+}
+
+template <int BM, int BN, int WM>
+int gemm_big_launch(const uint16_t* X, const uint16_t* W, void* Y, bool y_f32, bool accum, int M, int N, int K, int ldy,
+                    hipStream_t s) {
+    const unsigned grid = ceil_div((size_t)M, BM) * ceil_div((size_t)N, BN);
+    if (y_f32) {
+        if (accum) gemm_big<BM, BN, WM, kOutF32, true><<<grid, 512, 0, s>>>(X, W, Y, M, N, K, ldy);
+        else gemm_big<BM, BN, WM, kOutF32, false><<<grid, 512, 0, s>>>(X, W, Y, M, N, K, ldy);
+    } else {
+        if (accum) gemm_big<BM, BN, WM, kOutF16, true><<<grid, 512, 0, s>>>(X, W, Y, M, N, K, ldy);
+        else gemm_big<BM, BN, WM, kOutF16, false><<<grid, 512, 0, s>>>(X, W, Y, M, N, K, ldy);
+    }
+    return launch_status();
+}
+
+template <int BM, int BN, int WM>
+int gemm_big_silu_launch(const uint16_t* X, const uint16_t* W, void* Y, int M, int F, int K, int ldy, hipStream_t s) {
+    const unsigned grid = ceil_div((size_t)M, BM) * ceil_div((size_t)F, BN / 2);
+    gemm_big<BM, BN, WM, kOutSilu, false><<<grid, 512, 0, s>>>(X, W, Y, M, 2 * F, K, ldy);
     return launch_status();
 }
 
@@ -295,6 +495,10 @@ constexpr double kStageUs = 0.1;           // per 64-wide K stage
 constexpr double kCuBytesPerUs = 2.0e5;    // ~200 GB/s of operand tiles per CU
 constexpr double kCuFlopsPerUs = 8.0e6;    // ~8 TFLOP/s of fp16 MFMA per CU
 
+// Plain products of fewer stages stay on the ring's menu, whose tiles the existing callers of the tile
+// query rely on there (4096 x 4096 x 256, fp32 out: ring 27.5 us, 256 x 256 21.7).
+constexpr int kBigMinStages = 5;
+
 Tile pick_tile(int M, int N, int K, int cus, bool silu = false) {
     Tile best = {0, 0};
     double best_t = 1e300;
@@ -315,6 +519,42 @@ Tile pick_tile(int M, int N, int K, int cus, bool silu = false) {
     return best;
 }
 
+// The large-product tile a shape takes, or {0, 0} for the ring tile `t` of the menu. Times in us of a
+// round of one workgroup per CU, fitted to a sweep of both tiles and the ring over M 200 .. 4096 at
+// N x K of 768 x 768 .. 8192 x 4096 (14 pairs; fill: share of the CUs the tiles occupy, at most 1): a
+// tile's prologue and epilogue, then its stages. The estimate picked the faster side at each sweep
+// point beyond 4 %; small products stay on the ring (512 x 8192 x 4096: ring 45.9, 256 x 128 78.9).
+Tile pick_big(int M, int N, int K, int cus, bool silu, const Tile& t) {
+    const int nk = K / kBK;
+    if (nk < (silu ? 2 : kBigMinStages)) return Tile{0, 0};
+    auto rounds = [&](const Tile& x, int per_cu) {
+        return ceil((double)ceil_div((size_t)M, x.bm) * ceil_div((size_t)N, x.bn) / ((double)cus * per_cu));
+    };
+    const int lds = ring_stages(t.bm, t.bn) * (t.bm + t.bn) * kRowBytes;
+    const double wg = nk * kStageUs + (double)(t.bm + t.bn) * K * 2 / kCuBytesPerUs +
+                      2.0 * t.bm * t.bn * K / kCuFlopsPerUs;
+    double best = 0.95 * rounds(t, (160 * 1024) / lds >= 2 ? 2 : 1) * (1.2 * wg + 3.0);
+    Tile r = {0, 0};
+    struct Big { Tile t; double fixed, stage, stage_full; };
+    constexpr Big kBig[] = {{{256, 256}, 6.0, 1.2, 0.42}, {{256, 128}, 4.5, 0.75, 0.33}};
+    for (const Big& b : kBig) {
+        const double fill = std::min(1.0, (double)ceil_div((size_t)M, b.t.bm) * ceil_div((size_t)N, b.t.bn) / cus);
+        const double est = rounds(b.t, 1) * (b.fixed + nk * (b.stage + b.stage_full * fill));
+        if (est < best) {
+            best = est;
+            r = b.t;
+        }
+    }
+    return r;
+}
+
+// The tile of cdna4_gemm_f16_nt (or, silu, of cdna4_gemm_f16_nt_silu; N counts gate and up rows).
+Tile choose_tile(int M, int N, int K, int cus, bool silu) {
+    const Tile t = pick_tile(M, N, K, cus, silu);
+    const Tile big = pick_big(M, N, K, cus, silu, t);
+    return big.bm ? big : t;
+}
+
 }  // namespace
 
 // Returns -1, launching nothing, for a shape this kernel does not take (K not a multiple of 64,
@@ -332,7 +572,7 @@ int llm_gemm_f16(const uint16_t* X, const uint16_t* W, void* Y, bool y_f32, bool
     if (((uintptr_t)X | (uintptr_t)W) % 16 || (uintptr_t)Y % (y_f32 ? 16 : 8)) return -1;
     if ((uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)N * K * 2 >= (1ull << 32)) return -1;   // 32-bit copy offsets
     const int cus = device_cus() > 0 ? device_cus() : 256;
-    Tile t = pick_tile(M, N, K, cus);
+    Tile t = choose_tile(M, N, K, cus, false);
     if (cold && t.bm == 32 && t.bn == 32 && M >= 64 &&
         (double)ceil_div((size_t)M, 64) * ceil_div((size_t)N, 32) <= 2.0 * cus)
         t = Tile{64, 32};
@@ -340,6 +580,8 @@ int llm_gemm_f16(const uint16_t* X, const uint16_t* W, void* Y, bool y_f32, bool
     if (t.bm == a && t.bn == b) return gemm_launch<a, b>(X, W, Y, y_f32, accum, M, N, K, ldy, s);
     CDNA4_GEMM_TILE(32, 32) CDNA4_GEMM_TILE(64, 32) CDNA4_GEMM_TILE(64, 64) CDNA4_GEMM_TILE(64, 96)
     CDNA4_GEMM_TILE(64, 128) CDNA4_GEMM_TILE(128, 64) CDNA4_GEMM_TILE(128, 96) CDNA4_GEMM_TILE(128, 128)
+    if (t.bm == 256 && t.bn == 256) return gemm_big_launch<256, 256, 2>(X, W, Y, y_f32, accum, M, N, K, ldy, s);
+    if (t.bm == 256 && t.bn == 128) return gemm_big_launch<256, 128, 4>(X, W, Y, y_f32, accum, M, N, K, ldy, s);
 #undef CDNA4_GEMM_TILE
     return -1;
 }
@@ -388,10 +630,12 @@ int llm_gemm_f16_silu(const uint16_t* X, const uint16_t* W, void* Y, int M, int 
     if (M <= 0 || F <= 0 || K <= 0 || K % kKMul || F % 4 || ldy % 4 || ldy < F) return -1;
     if (((uintptr_t)X | (uintptr_t)W) % 16 || (uintptr_t)Y % 8) return -1;
     if ((uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)2 * F * K * 2 >= (1ull << 32)) return -1;
-    const Tile t = pick_tile(M, 2 * F, K, device_cus() > 0 ? device_cus() : 256, true);
+    const Tile t = choose_tile(M, 2 * F, K, device_cus() > 0 ? device_cus() : 256, true);
 #define CDNA4_GEMM_TILE(a, b) \
     if (t.bm == a && t.bn == b) return gemm_silu_launch<a, b>(X, W, Y, M, F, K, ldy, s);
     CDNA4_GEMM_TILE(64, 64) CDNA4_GEMM_TILE(64, 128) CDNA4_GEMM_TILE(128, 64) CDNA4_GEMM_TILE(128, 128)
+    if (t.bm == 256 && t.bn == 256) return gemm_big_silu_launch<256, 256, 2>(X, W, Y, M, F, K, ldy, s);
+    if (t.bm == 256 && t.bn == 128) return gemm_big_silu_launch<256, 128, 4>(X, W, Y, M, F, K, ldy, s);
 #undef CDNA4_GEMM_TILE
     return -1;
 }
@@ -410,7 +654,7 @@ extern "C" int cdna4_gemm_f16_nt_silu(const void* X, const void* W, void* Y, int
 
 extern "C" int cdna4_gemm_f16_nt_silu_tile(int M, int F, int K, int* bm, int* bn) {
     if (M <= 0 || F <= 0 || K <= 0 || !bm || !bn) return CDNA4_ERR_INVALID_VALUE;
-    const cdna4::Tile t = cdna4::pick_tile(M, 2 * F, K, cdna4::device_cus() > 0 ? cdna4::device_cus() : 256, true);
+    const cdna4::Tile t = cdna4::choose_tile(M, 2 * F, K, cdna4::device_cus() > 0 ? cdna4::device_cus() : 256, true);
     *bm = t.bm;
     *bn = t.bn;
     return 0;
@@ -418,7 +662,7 @@ extern "C" int cdna4_gemm_f16_nt_silu_tile(int M, int F, int K, int* bm, int* bn
 
 extern "C" int cdna4_gemm_f16_nt_tile(int M, int N, int K, int* bm, int* bn) {
     if (M <= 0 || N <= 0 || K <= 0 || !bm || !bn) return CDNA4_ERR_INVALID_VALUE;
-    const cdna4::Tile t = cdna4::pick_tile(M, N, K, cdna4::device_cus() > 0 ? cdna4::device_cus() : 256);
+    const cdna4::Tile t = cdna4::choose_tile(M, N, K, cdna4::device_cus() > 0 ? cdna4::device_cus() : 256, false);
     *bm = t.bm;
     *bn = t.bn;
     return 0;
