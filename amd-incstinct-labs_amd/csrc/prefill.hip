@@ -5,7 +5,9 @@
 // sqrt(D)) V per (batch, query head), query head h reads kv head h / (nQH / nKVH), causal
 // mask "key > query -> excluded", fp32 softmax and accumulation, O / l with an l > 0 guard.
 //
-// MI355X design of the f16 / bf16 kernels (fa_pipe for large problems, fa_mfma for mid-size):
+// MI355X design of the f16 / bf16 kernels (fa_pipe for large problems, fa_mfma_keys below that, with
+// the keys of a query block split over the waves, fa_small for the smallest; fa_mfma for many short
+// causal sequences at D = 64; plan_mfma estimates each and takes the least):
 //   * S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_16x16x32_{f16,bf16}. In that orientation
 //     the S^T accumulator of a lane holds one query column (q = lane % 16) and 4 keys, so
 //     the softmax state (m, l) and the O^T accumulator of a query live in the same lanes:
@@ -18,7 +20,7 @@
 //     lanes that hold the same query (lanes q, q+16, q+32, q+48): two permlane swaps, only
 //     when some score exceeds the lazily kept reference maximum by more than kTau.
 //   * K and V tiles go HBM -> LDS with global_load_lds_dwordx4 (asynchronous, no VGPRs),
-//     a tile or two ahead of their use (fa_mfma: two buffers; fa_pipe: a ring of three). The
+//     a tile or two ahead of their use (fa_mfma: two buffers; the others: rings). The
 //     16-byte chunks of a key row are XOR-swizzled so the K operand reads (ds_read_b128) and
 //     the V^T operand reads (ds_read_b64_tr_b16) are both free of bank conflicts.
 //   * fa_pipe software-pipelines the key loop: the exponentials of one 32-key chunk are
@@ -29,6 +31,7 @@
 // The fp32 kernel (fa_f32) serves the fp32 arm of the reference configuration (fp32 in and
 // out, accuracy 1e-4) on the fp32 matrix-core instruction (v_mfma_f32_16x16x4_f32).
 #include <type_traits>
+#include <algorithm>
 
 #include "attn_tile.hpp"
 #include "attn_stream.hpp"
@@ -66,7 +69,7 @@ struct PrefillArgs {
     long long q_bs, q_hs, q_rs, k_bs, k_hs, k_rs, o_bs, o_hs, o_rs;
     int seqQ, seqK, nQH, nKVH, batch, causal;
     int nqb;          // q blocks per (batch, head)
-    int xcd_map;      // 1: all q blocks of a (batch, head) on one XCD, heads in sequence
+    int xcd_map;      // 1: all q blocks of a (batch, head) on one XCD, heads in sequence (fa_pipe: persistent_item's order)
     int copy32;       // 1: a K/V tile's rows span < 4 GiB (32-bit per-lane copy offsets)
     float sc;         // log2(e) / sqrt(D)
 };
@@ -474,11 +477,11 @@ __device__ __forceinline__ void pipe_region(const char* Kn, int kcn, const char*
 #pragma unroll
         for (int t = 0; t < QT; ++t) sn[t][i & 1] = mfma<kBf16>(ka[i], qb[t][i >> 1], sn[t][i & 1]);
         if (i + kAhead < NK) kread(i + kAhead);
-        // one copy of the next-but-one tile per odd slot (NK / 2 = 2 NI slots): the waves' copies
-        // then reach the texture unit spread over the region instead of all after the barrier
+        // the region's 2 NI copies spread over its NK slots (fa_pipe: one per odd slot): the waves'
+        // copies then reach the texture unit spread over the region instead of all after the barrier
         if constexpr (kCopy) {
-            static_assert(NK / 2 == 2 * NI, "one copy per odd slot");
-            if (i & 1) cp.issue(i >> 1);
+#pragma unroll
+            for (int c = i * 2 * NI / NK; c < (i + 1) * 2 * NI / NK; ++c) cp.issue(c);
         }
 #pragma unroll
         for (int v = 0; v < SL; ++v) soft(i * SL + v);
@@ -567,25 +570,31 @@ __device__ __forceinline__ void copy_tile_full(const uint16_t* head, long long r
     for (int j = 0; j < NI; ++j) stream::dma16_s(base, voff[j], tile + (j * W + wave) * 64 * 8);
 }
 
-// Work item of a persistent workgroup: item = round * gridDim.x + position. With xcd_map (grid
-// and batch * heads multiples of 8) the XCD of position p is p % 8 and it owns heads x, x + 8, ...;
-// the G = grid / 8 workgroups of an XCD take, in round r, G consecutive entries of that XCD's
-// head-major, heaviest-first item list (so they share one or a few heads' K/V in the XCD's L2),
-// and take them in reverse order on odd rounds, so that a workgroup that drew a heavy causal q
-// block in one round draws a light one in the next whatever the ratio of q blocks per head to G.
-// Without xcd_map: heads vary fastest, q blocks heaviest first.
-__device__ __forceinline__ void persistent_item(int item, int nqb, int nbh, int xcd_map, int& bh, int& qrev) {
-    if (xcd_map) {
-        const int grid = (int)gridDim.x;
-        const int r = item / grid, p = item - r * grid;
-        const int xcd = p & 7, sp = p >> 3, G = grid >> 3;
-        const int K = min(G, ((nbh * nqb) >> 3) - r * G);   // this round's entries per XCD
-        const int idx = r * G + ((r & 1) ? K - 1 - sp : sp);
-        bh = (idx / nqb) * 8 + xcd;
-        qrev = idx % nqb;
+// Work item of a persistent workgroup: item = round * grid + position, position = blockIdx.x. A group
+// of G = grid / X workgroups (X = 8 with order 1 or 2: the workgroups of an XCD, position % 8, which
+// own heads x, x + 8, ..; X = 1 with order 0) takes, in round r, G consecutive entries of its item
+// list, in reverse order on odd rounds, so that a workgroup that drew a heavy causal q block in one
+// round draws a light one in the next. The list is
+//   order 1: head-major, heaviest block first within a head: the workgroups of an XCD share one or a
+//            few heads' K/V in its L2;
+//   order 2 (and 0): heaviest blocks of all heads first, heads fastest: the rounds pair evenly whatever
+//            the ratio of q blocks per head to G.
+// The launcher adds up both orders' workgroup loads (pipe_load) and takes order 2 where it is ahead by
+// more than the sharing is worth.
+__host__ __device__ __forceinline__ void persistent_item(int item, int grid, int nqb, int nbh, int order, int& bh,
+                                                         int& qrev) {
+    const int sh = order ? 3 : 0;
+    const int r = item / grid, p = item - r * grid;
+    const int x = p & ((1 << sh) - 1), sp = p >> sh, G = grid >> sh, H = nbh >> sh;
+    const int left = H * nqb - r * G, K = left < G ? left : G;   // this round's entries
+    const int idx = r * G + ((r & 1) ? K - 1 - sp : sp);
+    if (order == 1) {
+        const int hh = idx / nqb;
+        qrev = idx - hh * nqb;
+        bh = (hh << sh) + x;
     } else {
-        bh = item % nbh;
-        qrev = item / nbh;
+        qrev = idx / H;
+        bh = ((idx - qrev * H) << sh) + x;
     }
 }
 
@@ -612,7 +621,7 @@ __global__ __launch_bounds__(64 * W) void fa_pipe(PrefillArgs a) {
     struct Item { int b, h, q0, qw0; };
     auto item_of = [&](int item) {
         int bh, qrev;
-        persistent_item(item, a.nqb, nbh, a.xcd_map, bh, qrev);
+        persistent_item(item, (int)gridDim.x, a.nqb, nbh, a.xcd_map, bh, qrev);
         const int qblk = a.causal ? (a.nqb - 1 - qrev) : qrev;
         Item it;
         it.b = bh / a.nQH;
@@ -780,6 +789,237 @@ __global__ __launch_bounds__(64 * W) void fa_pipe(PrefillArgs a) {
             }
         }
         __syncthreads();   // every wave is done with the LDS ring before the next item's copies
+    }
+}
+
+// ---- the keys of a query block split over the waves (fa_mfma_keys) ----------------------------
+// fa_pipe's regions with the waves of a workgroup as QG groups of 32 queries x KG groups of keys: a
+// step of the key loop is 32 KG keys, of which wave (qg, kg) takes 32-key chunk kg. A workgroup then
+// serves 32 QG queries, and a query block takes 1 / KG of the steps, at the MFMAs per LDS read of
+// fa_pipe: the heaviest causal block, which sets the time of a grid of one or two rounds, gets
+// shorter, the items are finer, and a problem with few queries still fills the chip.
+// One region per step and wave: region t does P and P.V of the wave's chunk of step t and S^T of its
+// chunk of step t + 1, so it reads V of step t and K of step t + 1. K and V have rings of A + 1 slots
+// of their own; region t issues the copies of K (t + 1 + A) and V (t + A) into the slots that region
+// t - 1 read last; one workgroup barrier per step. At the end the KG waves of a query group exchange
+// (m, l, O) through LDS, each finishing 1 / KG of the group's outputs.
+// What bounds it: at one or two rounds the heaviest item (~0.7 us per region alone, ~0.95 with the
+// chip full, 1.0-1.2 for the 128-key steps, whose copies are twice the bytes), then ~6 us per item of
+// first loads, masked tail regions and the exchange. Measured (us, D 128 causal, before: the four-wave
+// fa_mfma, fa_small at S 512): B1 32/8 heads S 1,531 fp16 50.2 -> 33.5, bf16 53.7 -> 33.8, S 1,024 27.1
+// -> 22.4, S 512 25.1 -> 12.1; H8 S 4,096 71 -> 47; B3 H4 S 2,014 85 -> 27; D 64 H12 S 2,048 41 -> 18.
+// One item per workgroup: a persistent form (next item's Q and K loaded over the exchange) took 39.2
+// where this takes 33.5: the light blocks' snake pairing costs more than the launches. A = 2 for
+// KG = 2: with three steps ahead the first fill is longer (33.5 / 34.3 f16, 33.7 / 33.8 bf16, level).
+template <int D, int KG, int A, bool kBf16>
+__global__ __launch_bounds__(512) void fa_mfma_keys(PrefillArgs a) {
+    constexpr int W = 8, QG = W / KG, QT = 2, NS = A + 1;
+    constexpr int ND = D / 32, NDT = D / 16;
+    constexpr int BM = QG * QT * 16;
+    constexpr int TK = 32 * KG;                        // keys per step
+    constexpr int kTile = TK * D;                      // elements of a step's K (or V)
+    constexpr int NI = TK * (D / 8) / (64 * W);        // copies per wave of a step's K (or V)
+    static_assert(NI >= 1 && QG >= 1, "");
+    constexpr int kPart = QT * NDT / KG;               // 16-row d tiles each wave finishes
+    constexpr int kXchg = W * (KG - 1) * kPart * 256;  // floats exchanged
+    constexpr int kRing = 2 * NS * kTile;              // elements: K slots, then V slots
+    static_assert(kXchg * 4 <= kRing * 2, "the exchange fits over the rings");
+    __shared__ __attribute__((aligned(16))) uint16_t lds[kRing];
+    __shared__ __attribute__((aligned(16))) float2 ml_s[W][QT][16];
+
+    const int lane = (int)(threadIdx.x & 63u);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int li = lane & 15, g = lane >> 4;
+    const int qg = wave % QG, kg = wave / QG;
+    uint16_t* const vring = lds + NS * kTile;
+
+    // One work item per workgroup, query blocks heaviest (causal) first and heads fastest: the heavy
+    // items start first and the light ones fill the CUs that finish; with batch x heads a multiple of
+    // 8 a head stays on one XCD (workgroups go to the XCDs round-robin).
+    const int nbh = a.batch * a.nQH;
+    const int qrev = (int)blockIdx.x / nbh, bh = (int)blockIdx.x - qrev * nbh;
+    const int b = bh / a.nQH, h = bh - b * a.nQH, kvh = h / (a.nQH / a.nKVH);
+    const int q0 = (a.causal ? (a.nqb - 1 - qrev) : qrev) * BM, qw0 = q0 + qg * QT * 16;
+    const uint16_t* Kh = a.K + b * a.k_bs + kvh * a.k_hs;
+    const uint16_t* Vh = a.V + b * a.k_bs + kvh * a.k_hs;
+    u32x4 qb[QT][ND];
+    {
+        const uint16_t* Qh = a.Q + b * a.q_bs + h * a.q_hs;
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            const int q = min(qw0 + t * 16 + li, a.seqQ - 1);
+#pragma unroll
+            for (int c = 0; c < ND; ++c) qb[t][c] = *(const u32x4*)(Qh + q * a.q_rs + c * 32 + g * 8);
+        }
+    }
+    int nst = (a.seqK + TK - 1) / TK;
+    if (a.causal) nst = min(nst, (min(q0 + BM, a.seqQ) - 1) / TK + 1);
+    // per-lane byte offsets of a whole step's copies from the step's first row (copy32)
+    uint32_t koff[NI], voff[NI];
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+        const int p = (j * W + wave) * 64 + lane, r = p / (D / 8), c = p % (D / 8);
+        koff[j] = (uint32_t)(((long long)r * a.k_rs + (c ^ swz_k<D>(r)) * 8) * 2);
+        voff[j] = (uint32_t)(((long long)r * a.k_rs + (c ^ swz_v<D>(r)) * 8) * 2);
+    }
+    auto copy = [&](const uint16_t* head, int t, auto is_k) {   // K or V of step t into its slot
+        constexpr bool kIsK = decltype(is_k)::value;
+        uint16_t* dst = (kIsK ? lds : vring) + (t % NS) * kTile;
+        if (a.copy32 && (t + 1) * TK <= a.seqK) {
+            const uint16_t* base = head + (long long)t * TK * a.k_rs;
+#pragma unroll
+            for (int j = 0; j < NI; ++j) stream::dma16_s(base, kIsK ? koff[j] : voff[j], dst + (j * W + wave) * 512);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NI; ++j) {
+                const int p = (j * W + wave) * 64 + lane, r = p / (D / 8), c = p % (D / 8);
+                const int key = min(t * TK + r, a.seqK - 1);   // rows past the end re-read the last key (masked)
+                stream::dma16(head + key * a.k_rs + (c ^ swz<D, kIsK>(r)) * 8, dst + (j * W + wave) * 512);
+            }
+        }
+    };
+    const float inv_sc = 1.f / a.sc;
+    f32x4 o[QT][NDT], lacc[QT];
+    float m[QT], thr[QT];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        m[t] = kInitM;
+        thr[t] = (kInitM + kTau) * inv_sc;
+        lacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < NDT; ++d) o[t][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    // Main steps t < t_main: every chunk of step t + 1 lies below the workgroup's first query and
+    // inside seqK, and the steps whose K and V region t copies exist and are whole.
+    int t_main = min(a.seqK / TK, nst) - 1 - A;
+    if (a.causal) t_main = min(t_main, q0 >= 2 * TK - 1 ? (q0 - (2 * TK - 1)) / TK + 1 : 0);
+    if (!a.copy32) t_main = 0;
+    const int wave_qmax = min(qw0 + QT * 16, a.seqQ) - 1;   // last real query of this wave (if any)
+    const int kend = a.causal ? min(a.seqK, wave_qmax + 1) : a.seqK;
+    const int nch = (kend + 31) / 32;                        // the wave's queries see chunks c < nch; kg takes c % KG == kg
+    // K 0, then in the order the regions wait for them: K 1 and V 0, K 2 and V 1, ..
+    copy(Kh, 0, std::true_type{});
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+        if (i + 1 < nst) copy(Kh, i + 1, std::true_type{});
+        if (i < nst) copy(Vh, i, std::false_type{});
+    }
+    // K of step 0 landed (K 1 .. A and V 0 .. A - 1 are newer)
+    if (nst > A) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * A * NI) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    __syncthreads();
+    // Operand offsets of the wave's chunk in a slot (a chunk is 32 D 2 bytes), V's from the V ring, so
+    // that a slot is an immediate of the reads.
+    LdsOffsets off = lds_offsets<D>(li, g);
+    off.k += (uint32_t)kg * (32 * D * 2);
+    off.v += (uint32_t)kg * (32 * D * 2) + NS * kTile * 2;
+
+    // S^T of the wave's chunk of step 0, its mask and max check
+    f32x4 s[QT][2];
+    qk_chunk<D, QT, kBf16>((const char*)lds, off, qb, s, 0);
+    {
+        const int kb = 32 * kg;
+        float lm[QT];
+        if (kb + 32 > a.seqK || (a.causal && kb + 31 > qw0)) mask_chunk<QT>(s, kb, qw0, a.seqK, a.causal, li, g);
+        const bool need = check_raw<QT>(s, thr, lm) && kg < nch;
+        if (__builtin_amdgcn_ballot_w64(need)) rescale_pipe<D, QT>(lm, m, thr, o, lacc, a.sc, inv_sc);
+    }
+    u32x4 ones;
+    {
+        const uint32_t one2 = kBf16 ? 0x3F803F80u : 0x3C003C00u;
+        ones = u32x4{one2, one2, one2, one2};
+        asm volatile("" : "+v"(ones));
+    }
+    auto region = [&](int t, auto tail, auto two, int slot) {   // slot: t % NS (a literal in the main loop)
+        constexpr bool kTail = decltype(tail)::value;
+        // K of step t + 1 and V of step t landed (the pairs of the next A - 1 regions are newer) and
+        // are visible; every wave is past region t - 1, the last reader of the slots that region t
+        // copies into.
+        if (kTail && t + A >= nst) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * (A - 1) * NI) : "memory");
+        __syncthreads();
+        if (kTail) {
+            if (t + 1 + A < nst) copy(Kh, t + 1 + A, std::true_type{});
+            if (t + A < nst) copy(Vh, t + A, std::false_type{});
+        }
+        const int s1 = slot == NS - 1 ? 0 : slot + 1, sv = slot == 0 ? NS - 1 : slot - 1;
+        const char* Kn = (const char*)(lds + s1 * kTile);
+        const char* Vc = (const char*)(lds + slot * kTile);
+        TileCopy<NI> cp{Kh + (long long)(t + 1 + A) * TK * a.k_rs, Vh + (long long)(t + A) * TK * a.k_rs,
+                        lds + slot * kTile, vring + sv * kTile, koff, voff, wave, W};
+        const int j = KG * t + kg;
+        if (!kTail)
+            pipe_region<D, QT, kBf16, false, true, NI>(Kn, 0, Vc, 0, off, qb, s, o, m, thr, lacc, ones, true,
+                                                       (j + KG) * 32, qw0, a.seqK, a.causal, a.sc, inv_sc, li, g, cp);
+        else if (j < nch)
+            pipe_region<D, QT, kBf16, true, false, NI, decltype(two)::value>(
+                Kn, 0, Vc, 0, off, qb, s, o, m, thr, lacc, ones, j + KG < nch, (j + KG) * 32, qw0, a.seqK, a.causal,
+                a.sc, inv_sc, li, g, cp);
+    };
+    constexpr int t0 = kBf16 ? 1 : 0;
+    if constexpr (kBf16) {   // keys below kLoKeys enter with their weights' second bf16 term
+        static_assert(TK >= kLoKeys, "in step 0");
+        region(0, std::true_type{}, std::true_type{}, 0);
+    }
+    int t = t0;
+    for (; t + NS <= t_main; t += NS) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) region(t + i, std::false_type{}, std::false_type{}, (t0 + i) % NS);
+    }
+    for (; t < nst; ++t) region(t, std::true_type{}, std::false_type{}, t % NS);
+
+    __syncthreads();   // every wave is done with the rings
+    // Part p of a query group's outputs (d tiles p kPart .. of the QT x NDT tiles, query tile first)
+    // is finished by the wave with kg = p: every wave leaves the other parts' O and its (m, l).
+    float* px = (float*)lds;
+    if (g == 0) {
+#pragma unroll
+        for (int x = 0; x < QT; ++x) ml_s[wave][x][li] = make_float2(m[x], lacc[x][0]);
+    }
+#pragma unroll
+    for (int p = 0; p < KG; ++p) {
+        if (p == kg) continue;
+        float* dst = px + ((wave * (KG - 1) + (p < kg ? p : p - 1)) * kPart) * 256 + lane * 4;
+#pragma unroll
+        for (int i = 0; i < kPart; ++i) *(f32x4*)(dst + i * 256) = o[(p * kPart + i) / NDT][(p * kPart + i) % NDT];
+    }
+    __syncthreads();
+    uint16_t* Oh = a.O + b * a.o_bs + h * a.o_hs;
+#pragma unroll
+    for (int p = 0; p < KG; ++p) {
+        if (p != kg) continue;
+        const int x = p * kPart / NDT;   // the part's query tile
+        float2 ml[KG];
+        float M = kInitM, lt = 0.f;
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+            ml[k] = ml_s[k * QG + qg][x][li];
+            M = fmaxf(M, ml[k].x);
+        }
+        f32x4 r[kPart];
+#pragma unroll
+        for (int i = 0; i < kPart; ++i) r[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+            const float wt = __builtin_amdgcn_exp2f(ml[k].x - M);
+            lt = fmaf(ml[k].y, wt, lt);
+            const float* src = px + (((k * QG + qg) * (KG - 1) + (p < k ? p : p - 1)) * kPart) * 256 + lane * 4;
+#pragma unroll
+            for (int i = 0; i < kPart; ++i) {
+                const f32x4 v = k == p ? o[(p * kPart + i) / NDT][(p * kPart + i) % NDT] : *(const f32x4*)(src + i * 256);
+                r[i] += v * wt;
+            }
+        }
+        const float inv = (lt > 0.f) ? 1.f / lt : 1.f;
+        const int q = qw0 + x * 16 + li;
+        if (q < a.seqQ) {
+#pragma unroll
+            for (int i = 0; i < kPart; ++i) {
+                const int dt = (p * kPart + i) % NDT;
+                *(u32x2*)(Oh + q * a.o_rs + dt * 16 + g * 4) =
+                    u32x2{pack2<kBf16>(r[i][0] * inv, r[i][1] * inv), pack2<kBf16>(r[i][2] * inv, r[i][3] * inv)};
+            }
+        }
     }
 }
 
@@ -1001,39 +1241,138 @@ __global__ __launch_bounds__(64 * W) void fa_small(PrefillArgs a) {
     }
 }
 
-// Kernel choice for the 16-bit path: the pipelined 8 waves x 32 queries (two waves per SIMD, one
-// workgroup per CU) once its 256-query blocks fill the CUs at least once (causal) or a quarter of
-// them (non-causal: every block has the same work, and one fast workgroup per block beat four-wave
-// workgroups of 64 queries at every size measured down to 64 blocks, e.g. B1 H8 S4096 622 -> 705
-// TFLOP/s; causal blocks below one round left the heaviest block on the critical path, e.g. B1 H12
-// S4096 603 -> 547); 4 waves x 16 queries for the remaining mid-size causal problems; for problems
-// whose 64-query blocks would not fill the CUs twice over, 16 queries per workgroup with the keys
-// split over its waves (the large form when one round of workgroups covers the grid).
-struct PrefillPlan { int kernel, waves, rows; long long grid; };
+// ---- kernel choice for the 16-bit path ---------------------------------------------------------
+// Five forms cover the range from a few rows to whole batches of long sequences; which is fastest
+// depends on how the items fill the CUs, so each is estimated and the least taken. An item of a form
+// costs `fixed` plus its steps times `step` (us, with the chip nearly idle), and `step` grows by up to
+// `load` as the work fills the chip (the clock falls with the power). The time is the larger of the
+// heaviest item and the CUs' share of all items (plus part of an item where they do not come out
+// even); fa_pipe's persistent workgroups are added up as they run. Constants fitted to sweeps of every
+// form (D 64 and 128, fp16 and bf16, causal and not, 1-64 heads x 1-8 batches, 32-8,192 queries and
+// keys): the pick was the fastest form measured, or within 5 % of it, at all but a few points. E.g.
+// (us, head-on) B1 32/8 heads S 1,531 D 128 causal: fa_mfma_keys<2> 33.5, <4> 40.6, fa_pipe 41.2, the
+// four-wave kernel 50.7; S 512: <4> 12.1, <2> 15.8, fa_pipe 19.7, fa_small 25.1; B1 H12 S 512 D 64:
+// <8> 7.4, <4> 8.2, fa_small 9.1; B1 H8 S 512 D 128: fa_small 9.2, <4> 10.9.
+enum PrefillForm { kFormPipe, kFormKeys2, kFormKeys4, kFormKeys8, kFormMfma4, kFormSmallL, kFormSmallS, kForms };
+struct FormCost { int rows, keys; double fixed, step, load; };   // queries per item, keys per step
+template <int D>
+constexpr FormCost form_cost(int f) {
+    constexpr bool d64 = D == 64;
+    switch (f) {
+        case kFormPipe: return d64 ? FormCost{256, 64, 4.5, 0.92, 0.22} : FormCost{256, 64, 5.5, 1.36, 0.28};
+        case kFormKeys2: return d64 ? FormCost{128, 64, 4.3, 0.50, 0.30} : FormCost{128, 64, 6.0, 0.70, 0.38};
+        case kFormKeys4: return d64 ? FormCost{64, 128, 3.4, 0.62, 0.15} : FormCost{64, 128, 5.0, 0.95, 0.15};
+        case kFormKeys8: return FormCost{32, 256, 2.8, 0.85, 0.10};      // D = 64 only
+        case kFormMfma4: return FormCost{64, 64, 2.5, 0.67, 0.00};       // D = 64 only
+        case kFormSmallL: return d64 ? FormCost{16, 256, 2.3, 0.66, 0.10} : FormCost{16, 128, 3.4, 0.90, 0.10};
+        default: return d64 ? FormCost{16, 128, 2.5, 1.10, 0.10} : FormCost{16, 64, 3.4, 1.00, 0.00};
+    }
+}
+
+struct PrefillPlan { int kernel, waves, rows; long long grid; int form, order; };
+
+// Steps of q block i (heaviest last) and of a whole head, blocks of `rows` queries, `keys` per step
+// (one a multiple of the other).
+long long block_steps(const cdna3_prefill_cfg& c, int rows, int keys, long long i) {
+    const long long k = c.causal ? std::min<long long>(c.seqK, (i + 1) * rows) : c.seqK;
+    return (k + keys - 1) / keys;
+}
+double head_steps(const cdna3_prefill_cfg& c, int rows, int keys, long long nqb) {
+    const double whole = (double)block_steps(c, rows, keys, nqb - 1);
+    if (!c.causal) return whole * nqb;
+    const long long n = nqb - 1;   // the blocks before the last are whole
+    if (rows >= keys) return whole + (double)(rows / keys) * n * (n + 1) / 2;
+    const long long k = keys / rows, g = n / k;
+    return whole + (double)k * g * (g + 1) / 2 + (double)(n - k * g) * (g + 1);
+}
+
+// Largest load of a persistent workgroup (us) under an order of persistent_item.
+double pipe_load(const cdna3_prefill_cfg& c, const FormCost& fc, double step, int grid, int nqb, int nbh, int order) {
+    const int X = order ? 8 : 1, items = nbh * nqb;
+    double worst = 0.0;
+    for (int p = 0; p < grid; p += X) {   // the XCDs' lists are alike: XCD 0
+        double t = 0.0;
+        for (int item = p; item < items; item += grid) {
+            int bh, qrev;
+            persistent_item(item, grid, nqb, nbh, order, bh, qrev);
+            t += fc.fixed * (item == p ? 1.0 : 0.6) + step * (double)block_steps(c, fc.rows, fc.keys, nqb - 1 - qrev);
+        }
+        worst = std::max(worst, t);
+    }
+    return worst;
+}
+
+constexpr long long kPipeSimItems = 1 << 15;       // larger grids: many rounds, taken as even
+constexpr double kPipeL2Bytes = 4.0 * 1024 * 1024; // an XCD's L2
 
 template <int D>
 PrefillPlan plan_mfma(const cdna3_prefill_cfg& c) {
     const long long heads = (long long)c.batch * c.nQHeads;
     const int cus = device_cus();
-    PrefillPlan p;
     const long long blocks8 = heads * ((c.seqQ + 255) / 256);
-    if (blocks8 >= (c.causal ? cus : cus / 4)) {
-        p.kernel = CDNA4_KERNEL_PREFILL_MFMA_8W; p.waves = 8; p.rows = 256;
-        p.grid = blocks8;
-        // One resident workgroup per CU at W = 8 (LDS and VGPRs allow no second), so a grid of one
-        // workgroup per CU (a multiple of 8, see the item mapping) runs every item without
-        // relaunch gaps between workgroups.
-        const int pcus = cus & ~7;
-        if (pcus >= 8 && p.grid > pcus) p.grid = pcus;
-    } else if (heads * ((c.seqQ + 63) / 64) >= 2LL * cus) {
-        p.kernel = CDNA4_KERNEL_PREFILL_MFMA_4W; p.waves = 4; p.rows = 64;
-        p.grid = heads * ((c.seqQ + 63) / 64);
-    } else {
-        p.kernel = CDNA4_KERNEL_PREFILL_SMALL; p.rows = 16;
-        p.grid = heads * ((c.seqQ + 15) / 16);
-        p.waves = small_waves<D>(p.grid <= cus);
+    PrefillPlan best{};
+    double best_t = 1e300;
+    for (int f = 0; f < kForms; ++f) {
+        if ((f == kFormKeys8 || f == kFormMfma4) && D != 64) continue;
+        if (f == kFormMfma4 && !c.causal) continue;
+        // fa_pipe gives the first keys their second bf16 term only where few keys are seen; below whole
+        // rounds (a quarter of one non-causal) the other forms, which always do, are as fast
+        if (f == kFormPipe && blocks8 < (c.causal ? cus : cus / 4)) continue;
+        const FormCost fc = form_cost<D>(f);
+        const long long nqb = (c.seqQ + fc.rows - 1) / fc.rows, items = heads * nqb;
+        if (f == kFormSmallL && items > cus) continue;
+        if (f == kFormSmallS && items <= cus) continue;
+        if (items > 0x7fffffffLL) continue;
+        const int slots = (f == kFormSmallS || f == kFormMfma4) ? 2 * cus : cus;   // workgroups resident at once
+        const double steps = head_steps(c, fc.rows, fc.keys, nqb) * heads;
+        const double heavy = (double)block_steps(c, fc.rows, fc.keys, nqb - 1);
+        const double util = std::min(1.0, (fc.fixed * items + fc.step * steps) / slots / (fc.fixed + fc.step * heavy));
+        const double step = fc.step * (1.0 + fc.load * util);
+        PrefillPlan p{};
+        p.form = f;
+        p.rows = fc.rows;
+        p.waves = f == kFormMfma4 ? 4 : (f == kFormSmallL || f == kFormSmallS) ? small_waves<D>(f == kFormSmallL) : 8;
+        p.grid = items;
+        double t;
+        if (f == kFormPipe) {
+            // One resident workgroup per CU (LDS and VGPRs allow no second), so a grid of one workgroup
+            // per CU (a multiple of 8, see persistent_item) runs every item without relaunch gaps.
+            const int pcus = cus & ~7;
+            if (pcus >= 8 && p.grid > pcus) p.grid = pcus;
+            p.order = heads % 8 == 0 && p.grid % 8 == 0 ? 1 : 0;
+            t = std::max(fc.fixed + step * heavy, (0.6 * fc.fixed * items + step * steps) / p.grid);
+            if (items > p.grid && items <= kPipeSimItems) {
+                t = pipe_load(c, fc, step, (int)p.grid, (int)nqb, (int)heads, p.order);
+                if (p.order == 1 && c.causal) {
+                    // order 2 costs K/V sharing once an XCD's heads outgrow its L2 (B4 H32 S 8,192 1,683 ->
+                    // 1,825 us at equal balance; B2 40/8 S 5,000 606 -> 510, B7 8/1 S 2,675 155 -> 117)
+                    const double kv = 4.0 * c.seqK * c.D * std::max(1.0, heads / 8.0 / (c.nQHeads / c.nKVHeads));
+                    const double t2 = pipe_load(c, fc, step, (int)p.grid, (int)nqb, (int)heads, 2);
+                    if (t2 * (kv > kPipeL2Bytes ? 1.08 : 1.03) < t) {
+                        t = t2;
+                        p.order = 2;
+                    }
+                }
+            }
+        } else {
+            // two fa_mfma workgroups of a CU slow each other's steps by half
+            t = (fc.fixed * items + step * (f == kFormMfma4 ? 1.5 : 1.0) * steps) / slots;
+            if (items > slots) t += (f == kFormMfma4 ? 0.15 : 0.4) * (fc.fixed + step * steps / items);
+            const double rounds = (f == kFormSmallL || f == kFormSmallS || c.causal) ? 1.0 : (double)((items + slots - 1) / slots);
+            t = std::max(t, rounds * (fc.fixed + step * heavy));
+        }
+        if (t < best_t) {
+            best_t = t;
+            best = p;
+        }
     }
-    return p;
+    // The reported kernel is the problem's size class (rows tells the form): whole rounds of 256-query
+    // blocks (a quarter of one when every block has the same work), 64-query blocks that fill the CUs
+    // twice, and the problems below that.
+    best.kernel = blocks8 >= (c.causal ? cus : cus / 4)              ? CDNA4_KERNEL_PREFILL_MFMA_8W
+                  : heads * ((c.seqQ + 63) / 64) >= 2LL * cus ? CDNA4_KERNEL_PREFILL_MFMA_4W
+                                                              : CDNA4_KERNEL_PREFILL_SMALL;
+    return best;
 }
 
 PrefillArgs make_args(const cdna3_prefill_cfg& c, const cdna3_prefill_strides& st, const void* Q, const void* K,
@@ -1056,24 +1395,24 @@ template <int D, bool kBf16>
 int dispatch_mfma(const cdna3_prefill_cfg& c, const cdna3_prefill_strides& st, const void* Q, const void* K,
                   const void* V, void* O, hipStream_t s) {
     const PrefillPlan p = plan_mfma<D>(c);
-    PrefillArgs a = make_args(c, st, Q, K, V, O, p.rows);
     const long long nbh = (long long)c.batch * c.nQHeads;
-    if (nbh * a.nqb > 0x7fffffffLL) return CDNA4_ERR_INVALID_VALUE;
-    switch (p.kernel) {
-        case CDNA4_KERNEL_PREFILL_MFMA_8W:
-            a.xcd_map = (nbh % 8 == 0) ? 1 : 0;
-            fa_pipe<D, 8, 2, kBf16><<<(unsigned)p.grid, 64 * 8, 0, s>>>(a);
-            break;
-        case CDNA4_KERNEL_PREFILL_MFMA_4W:
-            a.xcd_map = (nbh % 8 == 0) ? 1 : 0;
-            fa_mfma<D, 4, 1, kBf16><<<(unsigned)p.grid, 64 * 4, 0, s>>>(a);
-            break;
+    if (p.rows == 0) return CDNA4_ERR_INVALID_VALUE;   // more items than a grid holds
+    PrefillArgs a = make_args(c, st, Q, K, V, O, p.rows);
+    a.xcd_map = p.form == kFormPipe ? p.order : (nbh % 8 == 0) ? 1 : 0;
+    // 32-bit copy offsets of fa_mfma_keys: its steps are up to 256 rows
+    if (p.waves == 8 && p.rows < 256 && 256 * st.kv_row * 2 >= (1LL << 32)) a.copy32 = 0;
+    const unsigned grid = (unsigned)p.grid;
+    switch (p.form) {
+        case kFormPipe: fa_pipe<D, 8, 2, kBf16><<<grid, 512, 0, s>>>(a); break;
+        case kFormKeys2: fa_mfma_keys<D, 2, 2, kBf16><<<grid, 512, 0, s>>>(a); break;
+        case kFormKeys4: fa_mfma_keys<D, 4, 1, kBf16><<<grid, 512, 0, s>>>(a); break;
+        case kFormSmallL: fa_small<D, kBf16, small_waves<D>(true)><<<grid, 64 * small_waves<D>(true), 0, s>>>(a); break;
+        case kFormSmallS: fa_small<D, kBf16, small_waves<D>(false)><<<grid, 64 * small_waves<D>(false), 0, s>>>(a); break;
         default:
-            a.xcd_map = (nbh % 8 == 0) ? 1 : 0;
-            if (p.waves == small_waves<D>(true))
-                fa_small<D, kBf16, small_waves<D>(true)><<<(unsigned)p.grid, 64 * small_waves<D>(true), 0, s>>>(a);
-            else
-                fa_small<D, kBf16, small_waves<D>(false)><<<(unsigned)p.grid, 64 * small_waves<D>(false), 0, s>>>(a);
+            if constexpr (D == 64) {
+                if (p.form == kFormKeys8) fa_mfma_keys<64, 8, 1, kBf16><<<grid, 512, 0, s>>>(a);
+                else fa_mfma<64, 4, 1, kBf16><<<grid, 256, 0, s>>>(a);
+            }
     }
     return launch_status();
 }
