@@ -12,7 +12,8 @@
 //           publishes its aggregate, reads its predecessor groups' aggregates / prefixes 64
 //           at a time (one per lane) and writes the output. Every published word carries the
 //           call's epoch, so words left by earlier calls read as "not ready" and the flags need
-//           no clearing between calls. No LDS in either.
+//           no clearing between calls. Up to about two million elements (scan_layout::spread_u)
+//           single-wave tiles cover the chip and read all totals below them at once. No LDS.
 #include <type_traits>
 #include "common.hpp"
 #include <atomic>
@@ -220,8 +221,11 @@ int reduce_launch(const void* in, size_t n, void* out, void* ws, hipStream_t s) 
 // 1 KiB of contiguous lines (16-byte loads of 8 values left each lane's 32-byte output as two
 // stores 32 bytes apart, and the half-filled lines were written twice).
 using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
+typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
 template <int DT> struct ScanElem : Elem<DT> {
     using Load = u32x4;
+    using LoadU = u32x4_a4;   // at any element
     // A vector of the op's identity, for the vectors past the end of the last tile.
     template <class Op> __device__ static Load ident() {
         using Acc = typename Elem<DT>::Acc;
@@ -233,6 +237,7 @@ template <int DT> struct ScanElem : Elem<DT> {
 };
 template <int DT> struct ScanElem16 : Elem<DT> {
     using Load = u32x2;
+    using LoadU = u32x2_a2;
     static constexpr int VEC = 4;
     // Four packed copies of the op's identity (0, -inf for max, +inf for min), for the vectors past
     // the end of the last tile.
@@ -255,7 +260,7 @@ template <int DT> struct ScanElem16 : Elem<DT> {
 template <> struct ScanElem<CDNA4_F16> : ScanElem16<CDNA4_F16> {};
 template <> struct ScanElem<CDNA4_BF16> : ScanElem16<CDNA4_BF16> {};
 // Tile = 64 lanes x U vectors per lane (scan_layout::scan_u). The look-back costs about the same
-// per tile whatever its size, so tiles are as large as the register file allows at three waves per
+// per tile whatever its size, so the large tiles are as large as the register file allows at three waves per
 // SIMD (~155 VGPRs with the tile held as loaded): 32 16-byte vectors for 32- and 64-bit inputs (24 /
 // 36 / 40 ran 3-8 % slower), 64 8-byte vectors of four 16-bit values (48: 83 us, 64: 77 us, 80 at
 // two waves: 87 us at 2^26; held as fp32 values they had fitted 32, 83 us).
@@ -399,15 +404,14 @@ __device__ Acc look_back(const ScanState& st, size_t tile, Op op) {
 // 83 us, 64-bit 253 -> 202 us, and 200 -> 187 us with eight-wave groups).
 template <int DT> constexpr int scan_group_waves() { return scan_layout::scan_waves((int)sizeof(typename ScanElem<DT>::In)); }
 
-template <int DT, class Op, bool kVec>
-__global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_tiles(const void* __restrict__ in_, size_t n,
-                                                                          void* __restrict__ out_, ScanState st) {
+template <int DT, class Op, bool kVec, int U>
+__device__ __forceinline__ void scan_group(const void* __restrict__ in_, size_t n, void* __restrict__ out_,
+                                           const ScanState& st) {
     constexpr int kWaves = scan_group_waves<DT>();
     using E = ScanElem<DT>;
     using Acc = typename E::Acc;
     using Out = typename E::Out;
     constexpr int VEC = E::VEC;
-    constexpr int U = scan_u<DT, kVec>();
     constexpr size_t TILE = scan_layout::tile_elems(VEC, U);
     const typename E::In* in = (const typename E::In*)in_;
     Out* out = (Out*)out_;
@@ -426,12 +430,15 @@ __global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_tiles(const 
     Acc* s_tot = (Acc*)(st.xchg + group * scan_layout::kXchgStride);
     Acc* s_excl = s_tot + kWaves;
 
-    // Aligned calls (kVec): n counts the elements of whole VEC-element vectors only (the host
-    // scans the remaining n % VEC elements in scan_tail). Every tile but the last is full and
-    // takes a straight-line path of vector loads at fixed offsets from one base, all issued before
-    // any arithmetic; the last tile guards each vector with a 32-bit tile-local index against the
-    // uniform vector count. Misaligned calls go element by element.
-    // 16- and 64-bit inputs on the aligned path (kRaw) keep the tile in registers as loaded (16-bit
+    // Every tile but the last is full and takes a straight-line path of vector loads at fixed
+    // offsets from one base, all issued before any arithmetic; the last tile guards each vector with
+    // a 32-bit tile-local index against the uniform vector count. Aligned calls (kVec): n counts the
+    // elements of whole VEC-element vectors only (the host scans the remaining n % VEC elements in
+    // scan_tail). Otherwise vectors lie at any element, which the memory path takes at nearly the
+    // aligned rate (2^26: f32 106 against 100 us, f16 80 against 75, i64 186 against 186; element by
+    // element these were 182, 295 and 304), and the last tile's elements past its last whole vector
+    // go one by one.
+    // 16- and 64-bit inputs (kRaw) keep the tile in registers as loaded (16-bit
     // values packed, two VGPRs per four) while only its total is formed, a fold per lane and one
     // over the wave, so the group's aggregate goes out before the tile's scan is computed, after the
     // look-back; past the end of the last tile the vectors hold the op's identity. Packed 16-bit
@@ -439,7 +446,7 @@ __global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_tiles(const 
     // 64-bit 200 -> 198 us). 32-bit inputs hold the scanned values across the look-back instead,
     // so the stores follow it at once (held as loaded: f32 101.1 -> 101.8 us, i32 100.9 -> 103.0).
     const typename E::In* tin = in + base;
-    const bool full = live && kVec && scan_layout::tile_full(base, TILE, n);
+    const bool full = live && scan_layout::tile_full(base, TILE, n);
     const uint32_t rem = live ? scan_layout::tile_rem(base, TILE, n) : 0u;  // elements (0: none)
     // Local inclusive scan of one vector of VEC values per lane: within the lane, then across the
     // wave (DPP), carried on from `run`, the combined value of the tile's earlier vectors.
@@ -454,21 +461,36 @@ __global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_tiles(const 
         for (int e = 0; e < VEC; ++e) x[e] = op(pre, x[e]);
         run = op(run, wave::xlane::lane63(inc));             // chunk total, on every lane
     };
-    constexpr bool kRaw = kVec && sizeof(typename E::In) != 4;
+    constexpr bool kRaw = sizeof(typename E::In) != 4;
+    using Load = typename std::conditional<kVec, typename E::Load, typename E::LoadU>::type;
     typename E::Load r[kRaw ? U : 1];   // kRaw: the tile as loaded
     Acc v[kRaw ? 1 : U][VEC];           // otherwise: the tile's scanned values
     Acc run = id;                       // the tile's total, on every lane
     if constexpr (kRaw) {
-        const typename E::Load* src = (const typename E::Load*)tin + lane;
+        const Load* src = (const Load*)tin + lane;
         if (full) {
 #pragma unroll
             for (int j = 0; j < U; ++j) r[j] = __builtin_nontemporal_load(src + j * 64);
             __builtin_amdgcn_sched_barrier(0);
         } else {
 #pragma unroll
-            for (int j = 0; j < U; ++j)
-                r[j] = scan_layout::vec_live(false, j, lane, rem, VEC) ? __builtin_nontemporal_load(src + j * 64)
-                                                                      : E::template ident<Op>();
+            for (int j = 0; j < U; ++j) {
+                if (scan_layout::vec_live(false, j, lane, rem, VEC)) {
+                    r[j] = __builtin_nontemporal_load(src + j * 64);
+                } else {
+                    r[j] = E::template ident<Op>();
+                    if constexpr (!kVec) {   // the vector the last element falls into
+                        typename E::In part[VEC];
+                        __builtin_memcpy(part, &r[j], sizeof(r[j]));
+#pragma unroll
+                        for (int e = 0; e < VEC; ++e) {
+                            const uint32_t i = scan_layout::elem_in_tile(j, lane, e, VEC);
+                            if (i < rem) part[e] = tin[i];
+                        }
+                        __builtin_memcpy(&r[j], part, sizeof(r[j]));
+                    }
+                }
+            }
         }
         // For a float sum this total can differ from the last value of the scan after the look-back
         // by the rounding of the tile's total (a different order), which the next tiles then carry.
@@ -489,31 +511,24 @@ __global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_tiles(const 
 #pragma unroll
         for (int j = 0; j < U; ++j) asm volatile("" : "+v"(r[j]));
     } else {
-        if constexpr (kVec) {
-            const typename E::Load* src = (const typename E::Load*)tin + lane;
-            if (full) {
+        const Load* src = (const Load*)tin + lane;
+        if (full) {
 #pragma unroll
-                for (int j = 0; j < U; ++j) E::unpack(__builtin_nontemporal_load(src + j * 64), v[j]);
-                __builtin_amdgcn_sched_barrier(0);
-            } else {
+            for (int j = 0; j < U; ++j) E::unpack(__builtin_nontemporal_load(src + j * 64), v[j]);
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
 #pragma unroll
-                for (int j = 0; j < U; ++j) {
-                    if (scan_layout::vec_live(false, j, lane, rem, VEC)) {
-                        E::unpack(__builtin_nontemporal_load(src + j * 64), v[j]);
-                    } else {
+            for (int j = 0; j < U; ++j) {
+                if (scan_layout::vec_live(false, j, lane, rem, VEC)) {
+                    E::unpack(__builtin_nontemporal_load(src + j * 64), v[j]);
+                } else {
 #pragma unroll
-                        for (int e = 0; e < VEC; ++e) v[j][e] = id;
+                    for (int e = 0; e < VEC; ++e) {
+                        const uint32_t i = scan_layout::elem_in_tile(j, lane, e, VEC);
+                        v[j][e] = !kVec && i < rem ? E::load1(tin + i) : id;
                     }
                 }
             }
-        } else {
-#pragma unroll
-            for (int j = 0; j < U; ++j)
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    const uint32_t i = scan_layout::elem_in_tile(j, lane, e, VEC);
-                    v[j][e] = i < rem ? E::load1(tin + i) : id;
-                }
         }
 #pragma unroll
         for (int j = 0; j < U; ++j) scan_vec(v[j], run);
@@ -552,41 +567,52 @@ __global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_tiles(const 
     const Acc excl = op(*s_excl, wpre);
     if (!live) return;
     Out* tout = out + base;
-    if constexpr (kVec) {
-        constexpr int kWords = (int)(sizeof(Out) * VEC / 16);
-        u32x4* dst = (u32x4*)tout + lane * kWords;
-        Acc run2 = id;
+    constexpr int kWords = (int)(sizeof(Out) * VEC / 16);
+    using Store = typename std::conditional<kVec, u32x4, u32x4_a4>::type;
+    Store* dst = (Store*)tout + lane * kWords;
+    Acc run2 = id;
 #pragma unroll
-        for (int j = 0; j < U; ++j) {
-            Acc x[VEC];
-            if constexpr (kRaw) {   // the tile's scan, vector by vector from the loaded tile
-                E::unpack(r[j], x);
-                scan_vec(x, run2);
-            } else {
+    for (int j = 0; j < U; ++j) {
+        Acc x[VEC];
+        if constexpr (kRaw) {   // the tile's scan, vector by vector from the loaded tile
+            E::unpack(r[j], x);
+            scan_vec(x, run2);
+        } else {
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) x[e] = v[j][e];
-            }
-            if (scan_layout::vec_live(full, j, lane, rem, VEC)) {
-                Out o[VEC];
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) o[e] = (Out)op(excl, x[e]);
-#pragma unroll
-                for (int w = 0; w < kWords; ++w) {
-                    u32x4 q;
-                    __builtin_memcpy(&q, (const char*)o + 16 * w, 16);
-                    __builtin_nontemporal_store(q, dst + j * 64 * kWords + w);
-                }
-            }
+            for (int e = 0; e < VEC; ++e) x[e] = v[j][e];
         }
-    } else {
+        Out o[VEC];
 #pragma unroll
-        for (int j = 0; j < U; ++j)
+        for (int e = 0; e < VEC; ++e) o[e] = (Out)op(excl, x[e]);
+        if (scan_layout::vec_live(full, j, lane, rem, VEC)) {
+#pragma unroll
+            for (int w = 0; w < kWords; ++w) {
+                u32x4 q;
+                __builtin_memcpy(&q, (const char*)o + 16 * w, 16);
+                __builtin_nontemporal_store(q, dst + j * 64 * kWords + w);
+            }
+        } else if constexpr (!kVec) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const uint32_t i = scan_layout::elem_in_tile(j, lane, e, VEC);
-                if (i < rem) tout[i] = (Out)op(excl, v[j][e]);
+                if (i < rem) tout[i] = o[e];
             }
+        }
     }
+}
+
+// kVec: large tiles of aligned calls; otherwise the small tiles of mid-size calls of any alignment.
+template <int DT, class Op, bool kVec>
+__global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_tiles(const void* __restrict__ in_, size_t n,
+                                                                          void* __restrict__ out_, ScanState st) {
+    scan_group<DT, Op, kVec, scan_u<DT, kVec>()>(in_, n, out_, st);
+}
+
+// Large tiles of misaligned calls (small ones measured 111, 98 and 202 us at 2^26: f32, f16, i64).
+template <int DT, class Op>
+__global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_wide(const void* __restrict__ in_, size_t n,
+                                                                         void* __restrict__ out_, ScanState st) {
+    scan_group<DT, Op, false, scan_u<DT, true>()>(in_, n, out_, st);
 }
 
 // The last n % VEC (< VEC) elements of an aligned call, after scan_tiles has published every
@@ -613,12 +639,156 @@ __global__ __launch_bounds__(64) void scan_tail(const void* __restrict__ in_, si
     }
 }
 
+// ---- scan of small and mid sizes: single-wave tiles, one look-back over all of them ------------
+// Bound by launch and latency: a load, a store and one round trip through the slots. Up to
+// kSpreadTiles tiles of 64 x U vectors, one wave and workgroup each, so that a mid-size input
+// reaches every CU (groups of 32,768 fp32 elements leave a million on 31 of them) and a small one is
+// done by a few short waves. All tiles are resident together and publish their totals at about the
+// same time, so a tile does not walk back window by window: lane l of its wave reads the totals of
+// tiles l, l + 64, .. below it, all loads issued at once, until every one is there: one round trip
+// after the slowest. Vectors lie at any element; the last tile's elements go one by one (no tail
+// launch). Sizes and times: scan_layout::spread_u.
+using scan_layout::kSpreadTiles;
+
+template <int DT, class Op, int U>
+__global__ __launch_bounds__(64) void scan_spread(const void* __restrict__ in_, size_t n, void* __restrict__ out_,
+                                                  ScanState st) {
+    using E = ScanElem<DT>;
+    using Acc = typename E::Acc;
+    using Out = typename E::Out;
+    constexpr int VEC = E::VEC;
+    constexpr size_t TILE = scan_layout::tile_elems(VEC, U);
+    Op op;
+    const Acc id = Op::template identity<Acc>();
+    const unsigned lane = threadIdx.x;
+    const size_t tile = blockIdx.x, base = scan_layout::tile_base(tile, TILE);
+    const typename E::In* tin = (const typename E::In*)in_ + base;
+    Out* tout = (Out*)out_ + base;
+    const uint32_t rem = scan_layout::tile_rem(base, TILE, n);
+    const bool full = scan_layout::tile_full(base, TILE, n);
+    Acc v[U][VEC];
+    const typename E::LoadU* src = (const typename E::LoadU*)tin + lane;
+    if (full) {
+        typename E::Load r[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) r[j] = src[j * 64];
+#pragma unroll
+        for (int j = 0; j < U; ++j) E::unpack(r[j], v[j]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < U; ++j)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+                const uint32_t i = scan_layout::elem_in_tile(j, lane, e, VEC);
+                v[j][e] = i < rem ? E::load1(tin + i) : id;
+            }
+    }
+    Acc run = id;
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+#pragma unroll
+        for (int e = 1; e < VEC; ++e) v[j][e] = op(v[j][e - 1], v[j][e]);
+        Acc carry;
+        const Acc inc = scan_with_carry(v[j][VEC - 1], op, carry);
+        const Acc pre = op(run, dpp<kRowShr1>(carry, inc));
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[j][e] = op(pre, v[j][e]);
+        run = op(run, wave::xlane::lane63(inc));
+    }
+    if (gridDim.x > 1) publish(st.agg, tile, run, st.tag_agg);
+    if (tile == 0 && lane == 0) *st.epoch_word = st.epoch;   // scan status: the workspace's latest call
+    Acc excl = id;
+    if (tile > 0) {
+        constexpr int S = kSpreadTiles / 64;
+        Acc a[S];
+        uint32_t waiting = 0;   // slots of this lane not seen yet
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            a[s] = id;
+            if (lane + 64u * s < tile) waiting |= 1u << s;
+        }
+        for (uint32_t spin = 0;; ++spin) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                if (waiting & (1u << s)) {
+                    Acc x;
+                    if (read_slot<Acc>(st.agg, (long long)(lane + 64u * s), st.tag_agg, x)) {
+                        a[s] = x;
+                        waiting &= ~(1u << s);
+                    }
+                }
+            }
+            if (__ballot(waiting != 0u) == 0ull) break;
+            if (spin >= st.spin_limit) {
+                if (lane == 0) __hip_atomic_store(st.error, st.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s) excl = op(excl, a[s]);
+        excl = allreduce(excl, op);
+    }
+    if (full) {
+        constexpr int kWords = (int)(sizeof(Out) * VEC / 16);
+        u32x4_a4* dst = (u32x4_a4*)tout + lane * kWords;
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            Out o[VEC];
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) o[e] = (Out)op(excl, v[j][e]);
+#pragma unroll
+            for (int w = 0; w < kWords; ++w) {
+                u32x4 q;
+                __builtin_memcpy(&q, (const char*)o + 16 * w, 16);
+                dst[j * 64 * kWords + w] = q;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < U; ++j)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+                const uint32_t i = scan_layout::elem_in_tile(j, lane, e, VEC);
+                if (i < rem) tout[i] = (Out)op(excl, v[j][e]);
+            }
+    }
+}
+
+// Clears a captured call's slots: a graph's replays all carry the epoch of its capture, so the words
+// that one replay leaves would read as published in the next.
+__global__ __launch_bounds__(256) void scan_clear(uint64_t* __restrict__ words, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) words[i] = 0;
+}
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+        (void)hipGetLastError();   // not this call's error: its own launch reports what the stream refuses
+        return false;
+    }
+    return status == hipStreamCaptureStatusActive;
+}
+
+template <int DT, class Op>
+int spread_launch(int u, const void* in, size_t n, void* out, const ScanState& st, hipStream_t s) {
+    const unsigned tiles = (unsigned)scan_layout::tiles_for(n, ScanElem<DT>::VEC, u);
+    switch (u) {
+        case 2: scan_spread<DT, Op, 2><<<tiles, 64, 0, s>>>(in, n, out, st); break;
+        case 4: scan_spread<DT, Op, 4><<<tiles, 64, 0, s>>>(in, n, out, st); break;
+        case 8: scan_spread<DT, Op, 8><<<tiles, 64, 0, s>>>(in, n, out, st); break;
+        default: scan_spread<DT, Op, scan_layout::kSpreadMaxU><<<tiles, 64, 0, s>>>(in, n, out, st);
+    }
+    return launch_status();
+}
+
 template <int DT, bool kVec>
 size_t scan_tiles_for(size_t n) {
     return scan_layout::tiles_for(n, ScanElem<DT>::VEC, scan_u<DT, kVec>());
 }
 
-// Tile count the workspace is sized for: the misaligned (smaller) tiles', the larger count.
+// Tile count the workspace is sized for: the small tiles', the larger count.
 size_t scan_ntiles(size_t n, int dtype) {
     switch (dtype) {
         case CDNA4_F32: return scan_tiles_for<CDNA4_F32, false>(n);
@@ -641,12 +811,12 @@ int scan_launch(const void* in, size_t n, void* out, void* ws, hipStream_t s) {
     constexpr size_t VEC = ScanElem<DT>::VEC;
     if (n == 0) return 0;
     if (scan_tiles_for<DT, false>(n) > 0x7fffffffull) return CDNA4_ERR_INVALID_VALUE;
-    // 16-byte aligned calls scan the whole vectors in scan_tiles and the last n % VEC elements
-    // in scan_tail; misaligned calls scan everything element by element in scan_tiles.
-    const bool vec = ((uintptr_t)in % 16) == 0 && ((uintptr_t)out % 16) == 0;
-    const size_t n_main = scan_layout::main_elems(n, vec, (int)VEC);
-    const size_t ntiles = vec ? scan_tiles_for<DT, true>(n_main) : scan_tiles_for<DT, false>(n_main);
     constexpr int kWaves = scan_group_waves<DT>();
+    const int spread = scan_layout::spread_u(n, (int)VEC);
+    const bool large = scan_layout::large_tiles(n, (int)VEC, (int)sizeof(typename Elem<DT>::In));
+    const bool vec = large && ((uintptr_t)in % 16) == 0 && ((uintptr_t)out % 16) == 0;
+    const size_t n_main = scan_layout::main_elems(n, vec, (int)VEC);
+    const size_t ntiles = large ? scan_tiles_for<DT, true>(n_main) : scan_tiles_for<DT, false>(n_main);
     const size_t ngroups = scan_layout::groups_for(ntiles, kWaves);   // look-back slots: one per group
     char* w = (char*)ws;
     ScanState st;
@@ -659,13 +829,20 @@ int scan_launch(const void* in, size_t n, void* out, void* ws, hipStream_t s) {
     st.agg = (uint64_t*)(w + scan_layout::agg_offset());
     st.pre = (uint64_t*)(w + scan_layout::pre_offset(ngroups));
     st.xchg = (unsigned char*)w + scan_layout::xchg_offset(ngroups);
-    constexpr unsigned kThreads = 64 * kWaves;
-    if (ngroups > 0) {
-        if (vec)
-            scan_tiles<DT, Op, true><<<(unsigned)ngroups, kThreads, 0, s>>>(in, n_main, out, st);
-        else
-            scan_tiles<DT, Op, false><<<(unsigned)ngroups, kThreads, 0, s>>>(in, n_main, out, st);
+    const size_t slots = spread ? scan_layout::tiles_for(n, (int)VEC, spread) : ngroups;
+    if (slots > 1 && capturing(s)) {   // the agg words, and of groups the pre words behind them
+        const size_t words = spread ? slots * Words<Acc>::NW
+                                    : (size_t)(st.pre - st.agg) + slots * Words<Acc>::NW;
+        scan_clear<<<(unsigned)((words + 255) / 256), 256, 0, s>>>(st.agg, words);
     }
+    if (spread) return spread_launch<DT, Op>(spread, in, n, out, st, s);
+    constexpr unsigned kThreads = 64 * kWaves;
+    if (vec)
+        scan_tiles<DT, Op, true><<<(unsigned)ngroups, kThreads, 0, s>>>(in, n_main, out, st);
+    else if (large)
+        scan_wide<DT, Op><<<(unsigned)ngroups, kThreads, 0, s>>>(in, n_main, out, st);
+    else
+        scan_tiles<DT, Op, false><<<(unsigned)ngroups, kThreads, 0, s>>>(in, n_main, out, st);
     if (n_main < n) scan_tail<DT, Op><<<1, 64, 0, s>>>(in, n_main, n, out, st, ngroups);
     return launch_status();
 }

@@ -13,8 +13,8 @@ namespace scan_layout {
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // A tile is 64 lanes x U vectors of VEC elements. U on the aligned path: kScanU for 4- and 8-byte
-// inputs, twice that for 16-bit inputs (held packed, 8 bytes per vector); on the misaligned
-// (element-wise) path half of kScanU.
+// inputs, twice that for 16-bit inputs (held packed, 8 bytes per vector); the small tiles of
+// mid-size calls (vec false) half of kScanU.
 constexpr int kScanU = 32;
 constexpr int scan_u(int in_bytes, bool vec, int base = kScanU) { return vec ? (in_bytes == 2 ? 2 * base : base) : base / 2; }
 constexpr size_t tile_elems(int vec, int u) { return (size_t)64 * vec * u; }
@@ -24,16 +24,18 @@ constexpr size_t tiles_for(size_t n, int vec, int u) { return (n + tile_elems(ve
 // [agg slots: align256(nslots * 16)][pre slots: align256(nslots * 16)][exchange lines:
 // nslots * kXchgStride], two 64-bit words per slot and array (one used by 32-bit values), and per
 // group one 128-byte line in which its waves leave their tile totals and wave 0 the group's prefix
-// (W + 1 values of at most 8 bytes, W the group's waves). The library sizes it by the misaligned
-// path's tile count, which bounds the group count of either path.
+// (W + 1 values of at most 8 bytes, W the group's waves). The library sizes it by the small tiles'
+// count, which bounds the group count of either size (and holds spread_u's slots: at two vectors a
+// tile takes 16 bytes where a small tile of eight times its elements has 160).
 constexpr size_t kXchgStride = 128;
 constexpr size_t ws_bytes(size_t ntiles) { return 256 + 2 * align256(ntiles * 16) + align256(ntiles * kXchgStride); }
 constexpr size_t agg_offset() { return 256; }
 constexpr size_t pre_offset(size_t ntiles) { return 256 + align256(ntiles * 16); }
 constexpr size_t xchg_offset(size_t ntiles) { return pre_offset(ntiles) + align256(ntiles * 16); }
 
-// Aligned calls scan whole VEC-element vectors in the tiles and the last n % VEC elements in a
-// one-wave tail; misaligned calls scan everything element by element.
+// Aligned calls of large tiles scan whole VEC-element vectors in the tiles and the last n % VEC
+// elements in a one-wave tail; all others scan every element in the tiles (vectors at any element,
+// the last tile's incomplete vector element by element).
 constexpr size_t main_elems(size_t n, bool vec, int VEC) { return vec ? n - n % (size_t)VEC : n; }
 
 // Tile t starts at element t * TILE; the elements it covers (TILE, or fewer for the last tile).
@@ -48,7 +50,7 @@ constexpr uint32_t vec_in_tile(int j, unsigned lane) { return (uint32_t)j * 64 +
 constexpr bool vec_live(bool full, int j, unsigned lane, uint32_t rem, int VEC) {
     return full || vec_in_tile(j, lane) < rem / (uint32_t)VEC;
 }
-// Element e of vector j of a lane on the element-wise (misaligned) path, and its guard.
+// Element e of vector j of a lane, for the elements that no whole vector holds.
 constexpr uint32_t elem_in_tile(int j, unsigned lane, int e, int VEC) { return vec_in_tile(j, lane) * (uint32_t)VEC + e; }
 
 // Tiles run in workgroups of W waves, one tile per wave: wave w of workgroup g scans tile g W + w
@@ -63,6 +65,33 @@ constexpr int scan_waves(int in_bytes) { return in_bytes == 8 ? 8 : 4; }
 static_assert((kScanWavesMax + 1) * 8 <= (int)kXchgStride, "a group's exchange values fit its line");
 constexpr size_t groups_for(size_t ntiles, int waves) { return (ntiles + waves - 1) / waves; }
 constexpr size_t group_tile(size_t group, unsigned wave, int waves) { return group * waves + wave; }
+
+// Which form scans n elements (times at f32, f16, i64 on the MI355X, us).
+//
+// Up to kSpreadTiles tiles of kSpreadMaxU vectors: single-wave tiles over the whole chip with one
+// look-back over all of them (scan_spread). Vectors per lane: the fewest of 2, 4, 8 that need at
+// most one tile per CU, then 8 and 16 with up to two (262,144 f32: 256 tiles 4.1, 512 tiles 5.1;
+// 1,000,003 f32: 489 tiles of 8 vectors 6.9, 245 of 16 7.6). Against groups of large tiles:
+// 1,000 elements 6.1 -> 3.5, 11.8 -> 3.6, 8.2 -> 4.1; 1,000,003 12.4 -> 7.1, 18.2 -> 7.0, 18.8 -> 9.0.
+constexpr int kSpreadTiles = 512;
+constexpr int kSpreadMaxU = 16;
+constexpr int spread_u(size_t n, int VEC) {
+    constexpr size_t one = kSpreadTiles / 2;
+    return tiles_for(n, VEC, 2) <= one ? 2
+         : tiles_for(n, VEC, 4) <= one ? 4
+         : tiles_for(n, VEC, 8) <= 2 * one ? 8
+         : tiles_for(n, VEC, kSpreadMaxU) <= 2 * one ? kSpreadMaxU : 0;
+}
+// Above that large tiles from large_groups groups of them on, one and a half per CU, for 16-bit
+// inputs, whose small tiles are a quarter, one; small tiles below. Fewer groups leave CUs idle
+// (4,194,304 elements: 12.8 -> 10.9, 17.0 -> 9.7, 19.2 -> 14.9; 8,388,608: 17.7 -> 16.3, 18.2 ->
+// 13.9, 25.2 -> 25.4), more have fewer look-backs in large tiles (16,777,216: small 27.5, 24.3,
+// 51.0, large 25.8, 20.4, 48.0; just below the line, 12,000,000: small 21.2, 18.6, 38.3, large 21.4,
+// 19.1, 42.2).
+constexpr int large_groups(int in_bytes) { return in_bytes == 2 ? 256 : 384; }
+constexpr bool large_tiles(size_t n, int VEC, int in_bytes) {
+    return groups_for(tiles_for(n, VEC, scan_u(in_bytes, true)), scan_waves(in_bytes)) >= (size_t)large_groups(in_bytes);
+}
 
 // 64-bit word w of group (slot) t's slot (NW words per slot).
 constexpr size_t slot_word(size_t tile, int nw, unsigned w) { return tile * (size_t)nw + w; }

@@ -202,7 +202,8 @@ int cdna3_attn_decode_plan(const cdna3_decode_cfg* cfg, int dtype, int with_work
  * n == 0: reduce writes the operator's identity; scan writes nothing.
  * Workspace: >= the returned size. The scan's look-back flags carry a per-call epoch, so a
  * workspace needs no clearing between calls (one launch per call, plus a one-wave tail launch
- * for the last n % 4 elements of an aligned call). A zeroed workspace, or one last used by
+ * for the last n % 4 elements of a large aligned call). A captured call also clears its flags, so
+ * that every replay of the graph waits for its own. A zeroed workspace, or one last used by
  * another scan, is always safe; memory never written by a scan is accepted too, with the caveat
  * that a 64-bit word of it whose upper half happens to equal the call's 32-bit tag would be read
  * as published (so zero a fresh workspace once to rule that out).
