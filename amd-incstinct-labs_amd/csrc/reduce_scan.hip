@@ -5,7 +5,8 @@
 // they run over whole HBM arrays without a single LDS instruction:
 //   reduce: stage 1 streams the input with 16-byte loads, each wave folds its share in
 //           registers and combines its 64 lanes with the DPP/permlane butterfly, then
-//           writes one partial; stage 2 (one wave) folds the partials.
+//           writes one partial; stage 2 (one workgroup) folds the partials. Small inputs take
+//           one workgroup and one launch.
 //   scan:   one pass with decoupled look-back. Each wave scans a tile held in registers
 //           (per-lane serial + wave scan per 64x16-byte chunk); the four waves of a
 //           workgroup meet their tile totals in a line of the workspace, and the group
@@ -30,6 +31,12 @@ using wave::xlane::allreduce;
 using wave::xlane::scan_with_carry;
 using wave::xlane::dpp;
 using wave::xlane::kRowShr1;
+
+using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
+// Vectors at any element.
+typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
 
 // ---- element traits: 16-byte vector <-> accumulator values ------------------------
 template <int DT> struct Elem;
@@ -157,6 +164,20 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_stage1(const void* __re
 // after the workgroup barrier wave 0 folds those 16. Deterministic order, no LDS.
 constexpr int kReduce2Threads = 1024;
 
+// Folds one value per thread of a kReduce2Threads workgroup through `slots` (one per wave, in the
+// workspace) into *out_.
+template <class Acc, class Op>
+__device__ __forceinline__ void meet_waves(Acc* slots, Acc a, Op op, void* out_) {
+    a = allreduce(a, op);
+    if ((threadIdx.x & 63u) == 0) slots[threadIdx.x >> 6] = a;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        Acc v = (threadIdx.x < kReduce2Threads / 64) ? slots[threadIdx.x] : Op::template identity<Acc>();
+        v = allreduce(v, op);
+        if (threadIdx.x == 0) *(Acc*)out_ = v;
+    }
+}
+
 template <int DT, class Op>
 __global__ __launch_bounds__(kReduce2Threads) void reduce_stage2(void* __restrict__ part_, int count,
                                                                   void* __restrict__ out_) {
@@ -172,15 +193,49 @@ __global__ __launch_bounds__(kReduce2Threads) void reduce_stage2(void* __restric
         v[u] = i < count ? part[i] : id;
     }
     Acc a = op(op(op(v[0], v[1]), op(v[2], v[3])), op(op(v[4], v[5]), op(v[6], v[7])));
-    a = allreduce(a, op);
-    Acc* wave_vals = part + count;   // kReduce2Threads / 64 slots after the partials
-    if ((threadIdx.x & 63u) == 0) wave_vals[threadIdx.x >> 6] = a;
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        Acc v = (threadIdx.x < kReduce2Threads / 64) ? wave_vals[threadIdx.x] : id;
-        v = allreduce(v, op);
-        if (threadIdx.x == 0) *(Acc*)out_ = v;
+    meet_waves(part + count, a, op, out_);   // kReduce2Threads / 64 slots after the partials
+}
+
+// Small inputs, bound by launches: one instead of two. A single workgroup reads vectors at any element, kReduceUnroll1 per
+// thread in flight, and its waves meet as in stage 2.
+constexpr int kReduceUnroll1 = 8;
+
+template <int DT, class Op>
+__global__ __launch_bounds__(kReduce2Threads) void reduce_small(const void* __restrict__ in_, size_t n,
+                                                                 void* __restrict__ ws_, void* __restrict__ out_) {
+    using E = Elem<DT>;
+    using Acc = typename E::Acc;
+    using Load = typename std::conditional<sizeof(typename E::In) == 2, u32x4_a2, u32x4_a4>::type;
+    const typename E::In* in = (const typename E::In*)in_;
+    Op op;
+    const Acc id = Op::template identity<Acc>();
+    Acc acc[kReduceUnroll1];
+#pragma unroll
+    for (int u = 0; u < kReduceUnroll1; ++u) acc[u] = id;
+    const unsigned nvec = (unsigned)(n / E::VEC);
+    const Load* vin = (const Load*)in;
+    for (unsigned base = threadIdx.x; base < nvec; base += kReduceUnroll1 * kReduce2Threads) {
+        u32x4 v[kReduceUnroll1];
+        // past the end: the last vector again, not folded
+#pragma unroll
+        for (int u = 0; u < kReduceUnroll1; ++u) {
+            const unsigned i = base + u * kReduce2Threads;
+            v[u] = vin[i < nvec ? i : nvec - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < kReduceUnroll1; ++u) {
+            Acc x[E::VEC];
+            E::unpack(v[u], x);
+#pragma unroll
+            for (int e = 1; e < E::VEC; ++e) x[0] = op(x[0], x[e]);
+            if (base + u * kReduce2Threads < nvec) acc[u] = op(acc[u], x[0]);
+        }
     }
+    const unsigned i = nvec * E::VEC + threadIdx.x;   // the last n % VEC elements
+    if (i < n) acc[0] = op(acc[0], E::load1(in + i));
+#pragma unroll
+    for (int u = 1; u < kReduceUnroll1; ++u) acc[0] = op(acc[0], acc[u]);
+    meet_waves((Acc*)ws_, acc[0], op, out_);
 }
 
 unsigned reduce_blocks(size_t n, int vec, int unroll) {
@@ -195,9 +250,16 @@ template <int DT, class Op>
 int reduce_launch(const void* in, size_t n, void* out, void* ws, hipStream_t s) {
     using E = Elem<DT>;
     constexpr size_t kEsz = sizeof(typename E::In);
+    // Up to 16 vectors per thread in one workgroup's launch, 8 where 16-bit elements lie at odd
+    // ones (their vectors cost more): two launches 5.9 us at any such size, one 3.5 up to 256 KB and
+    // 5.5-6.9 at 384-512 KB; at odd 16-bit elements 5.1 at 128 KB, 8.4 at 192 KB.
+    const uintptr_t addr = (uintptr_t)in;
+    if (n <= (size_t)kReduce2Threads * (addr % 4 == 0 ? 16 : 8) * E::VEC) {
+        reduce_small<DT, Op><<<1, kReduce2Threads, 0, s>>>(in, n, ws, out);
+        return launch_status();
+    }
     // A misaligned input (elements at their natural alignment) splits into the elements up to the
     // first 16-byte boundary, folded in by the first threads, and an aligned vector body.
-    const uintptr_t addr = (uintptr_t)in;
     size_t head = 0;
     bool vec = addr % 16 == 0;
     if (!vec && addr % kEsz == 0) {
@@ -220,9 +282,6 @@ int reduce_launch(const void* in, size_t n, void* out, void* ws, hipStream_t s) 
 // each lane's fp32 output vector leaves as one 16-byte store and every store instruction writes
 // 1 KiB of contiguous lines (16-byte loads of 8 values left each lane's 32-byte output as two
 // stores 32 bytes apart, and the half-filled lines were written twice).
-using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
-typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
-typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
 template <int DT> struct ScanElem : Elem<DT> {
     using Load = u32x4;
     using LoadU = u32x4_a4;   // at any element
