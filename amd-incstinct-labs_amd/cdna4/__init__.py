@@ -205,12 +205,18 @@ def _check(rc: int, what: str) -> None:
         raise CDNA4Error(what, rc)
 
 
-def _stream(stream) -> ctypes.c_void_p:
+# Handles and addresses go to the library as plain ints (its functions declare c_void_p), and the
+# current stream's handle comes without a torch.cuda.Stream object around it: the calls' Python was
+# longer than their kernels (reduce of 8,191 fp32 elements: 7.7 -> 5.4 us back to back).
+def _stream(stream) -> int:
     if stream is None:
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     if isinstance(stream, torch.cuda.Stream):
-        return ctypes.c_void_p(stream.cuda_stream)
-    return ctypes.c_void_p(int(stream))
+        return stream.cuda_stream
+    return int(stream)
+
+
+_NO_STREAM = contextlib.nullcontext()   # holds no state: one serves every call
 
 
 def _on_stream(stream):
@@ -220,14 +226,14 @@ def _on_stream(stream):
     work ordered after the kernels that still use it; allocated on another stream, it could be
     reused and overwritten while they run."""
     if stream is None:
-        return contextlib.nullcontext()
+        return _NO_STREAM
     if not isinstance(stream, torch.cuda.Stream):
         stream = torch.cuda.ExternalStream(int(stream))
     return torch.cuda.stream(stream)
 
 
-def _ptr(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
 
 
 def _dev(*ts: torch.Tensor) -> None:
@@ -255,8 +261,9 @@ def prefill(Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, O: torch.Tensor, 
     dt = _dtype(Q)
     if not (K.dtype == V.dtype == O.dtype == Q.dtype):
         raise ValueError("Q, K, V, O must share one dtype")
-    nq = cfg.batch * cfg.nQHeads * cfg.seqQ * cfg.D
-    nk = cfg.batch * cfg.nKVHeads * cfg.seqK * cfg.D
+    batch, D = cfg.batch, cfg.D
+    nq = batch * cfg.nQHeads * cfg.seqQ * D
+    nk = batch * cfg.nKVHeads * cfg.seqK * D
     if Q.numel() < nq or O.numel() < nq or K.numel() < nk or V.numel() < nk:
         raise ValueError("tensor smaller than the configuration")
     _check(lib().cdna3_attn_prefill(_ptr(Q), _ptr(K), _ptr(V), _ptr(O), ctypes.byref(cfg), dt,
