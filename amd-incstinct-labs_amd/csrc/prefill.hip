@@ -1031,133 +1031,163 @@ __global__ __launch_bounds__(512) void fa_mfma_keys(PrefillArgs a) {
 //   S^T = K Q^T, step s: lane (r = L % 16, g = L / 16) supplies K[key r][g D/4 + s] and
 //                        Q[query r][g D/4 + s]; C: lane (r, g) holds keys 4g + i of query r.
 //   O^T = V^T P^T, step s (keys 4g + s): B is the lane's own P of key 4g + s; A for row block b is
-//                        V[key 4g + s][16 b + r]; C: lane (r, g) holds O[query r][16 b + 4 g + i].
-// A workgroup of kF32Waves waves serves 16 queries of one (batch, head); wave w takes the 16-key
-// chunks w, w + W, ... (the causal diagonal spreads over the waves), keeps a running base-2
-// (m, l, O), and the waves merge through LDS at the end. The next chunk's K and V are loaded
-// into registers while the current one is computed.
-constexpr int kF32Br = 16;      // queries per workgroup
-// Waves per workgroup: at the reference configuration (B1 H8 S512 D64, 256 workgroups) the
-// per-wave chain of chunks bounds the time; eight waves ran 46.4 TFLOP/s against 43.8 with four
-// and 41.6 with sixteen (the LDS merge grows).
+//                        V[key 4g + s][NB r + b] (NB = D / 16; which of the D rows a block holds is free
+//                        too); C: lane (r, g) holds O[query r][NB (4 g + i) + b].
+// A workgroup of kF32Waves waves serves QT tiles of 16 queries of one (batch, head); wave w takes the
+// 16-key chunks w, w + W, ... (the causal diagonal spreads over the waves), keeps a running base-2
+// (m, l, O) per tile, and the waves merge through LDS at the end. K of the next chunk is loaded while
+// the current one's O product runs, V while the next S product does; every load is 16 bytes.
+//
+// Bound by the fp32 matrix rate (154 TFLOP/s for a large product) once the grid fills the chip, below
+// that by the chain of a workgroup's chunks: B1 H8 S512 D64 12.3 -> 10.8 us (4-byte V loads and a
+// copy of V before), B2 H8 S4096 D64 767 -> 668 us, 103 TFLOP/s. Two tiles halve the K and V each
+// CU reads, which bounds D = 128 (same shape at D128: one 1,498, two 1,285 us, 107 TFLOP/s); at D =
+// 64 they leave two waves per SIMD instead of four and lose (714 against 668). All waves split the
+// keys: waves with queries of their own ran up to 116 TFLOP/s, but a single chain over 1,030 keys
+// rounds to 7.2e-7 relative against 4.5e-7 for eight merged ones. At the small configuration
+// four waves with two chunks per step took 11.2 us, eight with two or four chunks 11.7 and 11.3.
 constexpr int kF32Waves = 8;
 
-template <int D>
-__device__ __forceinline__ void f32_chunk_load(const float* __restrict__ Kh, const float* __restrict__ Vh, int kb,
-                                               int seqK, int r, int g, float (&kf)[D / 4], float (&vf)[4][D / 16]) {
-    constexpr int DS = D / 4;
-    const float* kp = Kh + (size_t)min(kb + r, seqK - 1) * D + g * DS;
-#pragma unroll
-    for (int s = 0; s < DS; s += 4) {
-        const float4 v = *(const float4*)(kp + s);
-        kf[s] = v.x; kf[s + 1] = v.y; kf[s + 2] = v.z; kf[s + 3] = v.w;
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const float* vp = Vh + (size_t)min(kb + 4 * g + s, seqK - 1) * D + r;
-#pragma unroll
-        for (int b = 0; b < D / 16; ++b) vf[s][b] = vp[16 * b];
-    }
-}
-
-template <int D>
+template <int D, int QT>
 __global__ __launch_bounds__(64 * kF32Waves) void fa_f32(const float* __restrict__ Q, const float* __restrict__ K,
                                                          const float* __restrict__ V, float* __restrict__ O, int seqQ,
                                                          int seqK, int nQH, int nKVH, int causal, int nqb, int xcd_map,
                                                          float sc) {
     constexpr int DS = D / 4, NB = D / 16;
-    __shared__ __attribute__((aligned(16))) float o_s[kF32Waves][kF32Br][D];
-    __shared__ float m_s[kF32Waves][kF32Br], l_s[kF32Waves][kF32Br];
-    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    __shared__ __attribute__((aligned(16))) float o_s[kF32Waves][16][D + 4];   // rows a bank quad apart
+    __shared__ float m_s[kF32Waves][16], l_s[kF32Waves][16];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     const int r = lane & 15, g = lane >> 4;
     int bh, qb;
     block_item(blockIdx.x, nqb, xcd_map, bh, qb);
+    if (causal) qb = nqb - 1 - qb;   // the longest first
     const int b = bh / nQH, h = bh % nQH;
     const int kvh = h / (nQH / nKVH);
-    const int q0 = qb * kF32Br;
+    const int q0 = qb * 16 * QT;
     const float* Qh = Q + ((size_t)b * nQH + h) * (size_t)seqQ * D;
     const float* Kh = K + ((size_t)b * nKVH + kvh) * (size_t)seqK * D;
     const float* Vh = V + ((size_t)b * nKVH + kvh) * (size_t)seqK * D;
-
-    float qf[DS];
-    {
-        const float* qp = Qh + (size_t)min(q0 + r, seqQ - 1) * D + g * DS;
-#pragma unroll
-        for (int s = 0; s < DS; s += 4) {
-            const float4 v = *(const float4*)(qp + s);
-            qf[s] = v.x; qf[s + 1] = v.y; qf[s + 2] = v.z; qf[s + 3] = v.w;
-        }
-    }
-    const int kend = causal ? min(seqK, q0 + kF32Br) : seqK;
-    const int qrow = q0 + r;
-    float m = kInitM, lpart = 0.f;
-    f32x4 o[NB];
-#pragma unroll
-    for (int bb = 0; bb < NB; ++bb) o[bb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    float kf[DS], vf[4][NB];
-    int kb = wave * 16;
-    if (kb < kend) f32_chunk_load<D>(Kh, Vh, kb, seqK, r, g, kf, vf);
-    for (; kb < kend; kb += 16 * kF32Waves) {
-        f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < DS; ++s) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s], qf[s], st, 0, 0, 0);
-        float vc[4][NB];
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int bb = 0; bb < NB; ++bb) vc[s][bb] = vf[s][bb];
-        const int kn = kb + 16 * kF32Waves;
-        if (kn < kend) f32_chunk_load<D>(Kh, Vh, kn, seqK, r, g, kf, vf);   // next chunk, in flight
-        float p[4];
-        float mx = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int key = kb + 4 * g + i;
-            p[i] = (key < kend && !(causal && key > qrow)) ? st[i] * sc : -INFINITY;
-            mx = fmaxf(mx, p[i]);
-        }
-        mx = cross_row_allreduce(mx, Max{});
-        const float mnew = fmaxf(m, mx);
-        const float alpha = exp2f(m - mnew);
-        float ps = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            p[i] = exp2f(p[i] - mnew);
-            ps += p[i];
-        }
-        lpart = lpart * alpha + ps;
-        m = mnew;
-#pragma unroll
-        for (int bb = 0; bb < NB; ++bb) o[bb] *= alpha;
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int bb = 0; bb < NB; ++bb) o[bb] = __builtin_amdgcn_mfma_f32_16x16x4f32(vc[s][bb], p[s], o[bb], 0, 0, 0);
-    }
-    const float l = cross_row_allreduce(lpart, Sum{});
-#pragma unroll
-    for (int bb = 0; bb < NB; ++bb) *(f32x4*)&o_s[wave][r][16 * bb + 4 * g] = o[bb];
-    if (g == 0) {
-        m_s[wave][r] = m;
-        l_s[wave][r] = l;
-    }
-    __syncthreads();
     float* Oh = O + ((size_t)b * nQH + h) * (size_t)seqQ * D;
-    for (int idx = (int)threadIdx.x; idx < kF32Br * D; idx += 64 * kF32Waves) {
-        const int q = idx / D, d = idx % D;
-        if (q0 + q >= seqQ) break;
-        float M = kInitM;
+    const int kend = causal ? min(seqK, q0 + 16 * QT) : seqK;
+
+    f32x4 kf[DS / 4], vf[4][NB / 4], qf[QT][DS / 4];
+    auto load_k = [&](int kb) {
+        const f32x4* kp = (const f32x4*)(Kh + (size_t)min(kb + r, seqK - 1) * D + g * DS);
 #pragma unroll
-        for (int w = 0; w < kF32Waves; ++w) M = fmaxf(M, m_s[w][q]);
-        float L = 0.f, acc = 0.f;
+        for (int s = 0; s < DS / 4; ++s) kf[s] = kp[s];
+    };
+    auto load_v = [&](int kb) {
 #pragma unroll
-        for (int w = 0; w < kF32Waves; ++w) {
-            const float wt = exp2f(m_s[w][q] - M);
-            L = fmaf(wt, l_s[w][q], L);
-            acc = fmaf(wt, o_s[w][q][d], acc);
+        for (int s = 0; s < 4; ++s) {
+            const f32x4* vp = (const f32x4*)(Vh + (size_t)min(kb + 4 * g + s, seqK - 1) * D + r * NB);
+#pragma unroll
+            for (int bb = 0; bb < NB / 4; ++bb) vf[s][bb] = vp[bb];
         }
-        Oh[(size_t)(q0 + q) * D + d] = L > 0.f ? acc / L : 0.f;
+    };
+    int kb = wave * 16;
+    if (kb < kend) {
+        load_k(kb);
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            const f32x4* qp = (const f32x4*)(Qh + (size_t)min(q0 + 16 * t + r, seqQ - 1) * D + g * DS);
+#pragma unroll
+            for (int s = 0; s < DS / 4; ++s) qf[t][s] = qp[s];
+        }
+        load_v(kb);
+    }
+    float m[QT], lpart[QT];
+    f32x4 o[QT][NB];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        m[t] = kInitM;
+        lpart[t] = 0.f;
+#pragma unroll
+        for (int bb = 0; bb < NB; ++bb) o[t][bb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (; kb < kend; kb += 16 * kF32Waves) {
+        f32x4 st[QT];
+#pragma unroll
+        for (int t = 0; t < QT; ++t) st[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < DS; ++s)
+#pragma unroll
+            for (int t = 0; t < QT; ++t)
+                st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s / 4][s % 4], qf[t][s / 4][s % 4], st[t], 0, 0, 0);
+        const int kn = kb + 16 * kF32Waves;
+        if (kn < kend) load_k(kn);
+        const bool edge = kb + 16 > kend || (causal && kb + 15 > q0);   // some key is masked for some query
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            const int qrow = q0 + 16 * t + r;
+            float mx = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                st[t][i] *= sc;
+                if (edge) {
+                    const int key = kb + 4 * g + i;
+                    if (key >= kend || (causal && key > qrow)) st[t][i] = -INFINITY;
+                }
+                mx = fmaxf(mx, st[t][i]);
+            }
+            mx = cross_row_allreduce(mx, Max{});
+            const float mnew = fmaxf(m[t], mx);
+            if (__ballot(mnew != m[t])) {   // otherwise every factor is 1
+                const float alpha = exp2f(m[t] - mnew);
+                lpart[t] *= alpha;
+#pragma unroll
+                for (int bb = 0; bb < NB; ++bb) o[t][bb] *= alpha;
+                m[t] = mnew;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) st[t][i] = exp2f(st[t][i] - mnew);
+            lpart[t] += (st[t][0] + st[t][1]) + (st[t][2] + st[t][3]);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+                for (int t = 0; t < QT; ++t)
+                    o[t][bb] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[s][bb / 4][bb % 4], st[t][s], o[t][bb], 0, 0, 0);
+        if (kn < kend) load_v(kn);
+    }
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {   // the waves' merge, 16 queries at a time
+        const float l = cross_row_allreduce(lpart[t], Sum{});
+        if (t > 0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int b4 = 0; b4 < NB / 4; ++b4) {
+                f32x4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = o[t][4 * b4 + e][i];
+                *(f32x4*)&o_s[wave][r][NB * (4 * g + i) + 4 * b4] = v;
+            }
+        if (g == 0) {
+            m_s[wave][r] = m[t];
+            l_s[wave][r] = l;
+        }
+        __syncthreads();
+        // two neighbouring floats per thread (O may start at any float)
+        for (int idx = (int)threadIdx.x * 2; idx < 16 * D; idx += 128 * kF32Waves) {
+            const int row = idx / D, d = idx % D;
+            if (q0 + 16 * t + row >= seqQ) break;
+            float M = kInitM;
+#pragma unroll
+            for (int w = 0; w < kF32Waves; ++w) M = fmaxf(M, m_s[w][row]);
+            float L = 0.f, acc0 = 0.f, acc1 = 0.f;
+#pragma unroll
+            for (int w = 0; w < kF32Waves; ++w) {
+                const float wt = exp2f(m_s[w][row] - M);
+                L = fmaf(wt, l_s[w][row], L);
+                acc0 = fmaf(wt, o_s[w][row][d], acc0);
+                acc1 = fmaf(wt, o_s[w][row][d + 1], acc1);
+            }
+            float* op = Oh + (size_t)(q0 + 16 * t + row) * D + d;
+            op[0] = L > 0.f ? acc0 / L : 0.f;
+            op[1] = L > 0.f ? acc1 / L : 0.f;
+        }
     }
 }
 
@@ -1438,6 +1468,31 @@ cdna3_prefill_strides contiguous_strides(const cdna3_prefill_cfg& c) {
     return st;
 }
 
+// Query tiles per workgroup of fa_f32: two at D = 128 once that leaves three workgroups per CU (768
+// causal ones of B1 H16 S1531: 130 against 139 us with one tile; 384 of H12 S1000: 93 against 72).
+int f32_tiles(const cdna3_prefill_cfg& c) {
+    const long long pairs = (long long)c.batch * c.nQHeads * ((c.seqQ + 31) / 32);
+    return c.D == 128 && pairs >= 3LL * device_cus() ? 2 : 1;
+}
+
+template <int D, int QT>
+int launch_f32(const cdna3_prefill_cfg& c, const void* Q, const void* K, const void* V, void* O, hipStream_t s) {
+    const int nqb = (c.seqQ + 16 * QT - 1) / (16 * QT);
+    const long long blocks = (long long)c.batch * c.nQHeads * nqb;
+    const float sc = kLog2e / sqrtf((float)c.D);
+    const int xcd = ((long long)c.batch * c.nQHeads % 8 == 0) ? 1 : 0;
+    fa_f32<D, QT><<<(unsigned)blocks, 64 * kF32Waves, 0, s>>>((const float*)Q, (const float*)K, (const float*)V,
+                                                              (float*)O, c.seqQ, c.seqK, c.nQHeads, c.nKVHeads,
+                                                              c.causal ? 1 : 0, nqb, xcd, sc);
+    return launch_status();
+}
+
+int dispatch_f32(const cdna3_prefill_cfg& c, const void* Q, const void* K, const void* V, void* O, hipStream_t s) {
+    if ((long long)c.batch * c.nQHeads * ((c.seqQ + 15) / 16) > 0x7fffffffLL) return CDNA4_ERR_INVALID_VALUE;
+    if (c.D == 64) return launch_f32<64, 1>(c, Q, K, V, O, s);
+    return f32_tiles(c) == 2 ? launch_f32<128, 2>(c, Q, K, V, O, s) : launch_f32<128, 1>(c, Q, K, V, O, s);
+}
+
 }  // namespace
 }  // namespace cdna4
 
@@ -1453,22 +1508,7 @@ extern "C" int cdna3_attn_prefill(const void* Q, const void* K, const void* V, v
         return CDNA4_ERR_INVALID_VALUE;
     if (int e = check_device()) return e;
     hipStream_t s = (hipStream_t)stream;
-    if (dtype == CDNA4_F32) {
-        const int nqb = (c.seqQ + kF32Br - 1) / kF32Br;
-        const long long blocks = (long long)c.batch * c.nQHeads * nqb;
-        if (blocks > 0x7fffffffLL) return CDNA4_ERR_INVALID_VALUE;
-        const float sc = kLog2e / sqrtf((float)c.D);
-        const int xcd = ((long long)c.batch * c.nQHeads % 8 == 0) ? 1 : 0;
-        if (c.D == 128)
-            fa_f32<128><<<(unsigned)blocks, 64 * kF32Waves, 0, s>>>((const float*)Q, (const float*)K, (const float*)V,
-                                                                    (float*)O, c.seqQ, c.seqK, c.nQHeads, c.nKVHeads,
-                                                                    c.causal ? 1 : 0, nqb, xcd, sc);
-        else
-            fa_f32<64><<<(unsigned)blocks, 64 * kF32Waves, 0, s>>>((const float*)Q, (const float*)K, (const float*)V,
-                                                                   (float*)O, c.seqQ, c.seqK, c.nQHeads, c.nKVHeads,
-                                                                   c.causal ? 1 : 0, nqb, xcd, sc);
-        return launch_status();
-    }
+    if (dtype == CDNA4_F32) return dispatch_f32(c, Q, K, V, O, s);
     const cdna3_prefill_strides st = contiguous_strides(c);
     const bool bf = dtype == CDNA4_BF16;
     if (c.D == 128)
@@ -1511,8 +1551,8 @@ extern "C" int cdna3_attn_prefill_plan(const cdna3_prefill_cfg* cfg, int dtype, 
     if (dtype == CDNA4_F32) {
         out->kernel = CDNA4_KERNEL_PREFILL_F32;
         out->waves = kF32Waves;
-        out->rows = kF32Br;
-        out->grid = (long long)c.batch * c.nQHeads * ((c.seqQ + kF32Br - 1) / kF32Br);
+        out->rows = 16 * f32_tiles(c);
+        out->grid = (long long)c.batch * c.nQHeads * ((c.seqQ + out->rows - 1) / out->rows);
     } else if (dtype == CDNA4_F16 || dtype == CDNA4_BF16) {
         const PrefillPlan p = c.D == 128 ? plan_mfma<128>(c) : plan_mfma<64>(c);
         out->kernel = p.kernel;
