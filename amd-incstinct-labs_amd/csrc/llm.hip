@@ -62,6 +62,12 @@ __global__ __launch_bounds__(256) void embed_gather(const uint16_t* __restrict__
 }
 
 // ---- a wave's share of one row ---------------------------------------------------------------
+// A load that stays where it is written: issued early and used late, in flight in between (the
+// compiler moves an ordinary load down to its use, where the wave then waits a memory round trip).
+__device__ __forceinline__ float load_early(const float* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // A row of K elements (K % 8 == 0) is C = K / 8 chunks of 8; lane l holds chunks c = l + 64 j for
 // j < J (zero past C). Every load is clamped to the row instead of branched around, so all of a
 // lane's loads are in flight together: one memory latency per kernel, not one per chunk.
@@ -130,17 +136,17 @@ __device__ __forceinline__ void row_stats(const f32x4 (&lo)[J], const f32x4 (&hi
 }
 
 // y = (x - mean) * inv * g (+ b) of element e of chunk j, in fp32.
-template <int J>
+template <bool kBeta, int J>
 __device__ __forceinline__ float normed(const f32x4 (&lo)[J], const f32x4 (&hi)[J], const u32x4 (&g)[J],
-                                        const u32x4 (&b)[J], bool has_b, int j, int e, float mean, float inv) {
+                                        const u32x4 (&b)[J], int j, int e, float mean, float inv) {
     float o = (elem(lo[j], hi[j], e) - mean) * inv * half_of(g[j], e);
-    if (has_b) o += half_of(b[j], e);
+    if constexpr (kBeta) o += half_of(b[j], e);
     return o;
 }
 
 // Y[r][:] = norm(X[r][:]) * w + b for the prompt path, one wave per row, stored fp16 (the
 // projection input). kLayer = two-pass LayerNorm, else RMSNorm.
-template <int J, bool kLayer>
+template <int J, bool kLayer, bool kBeta>
 __global__ __launch_bounds__(256) void norm_cast(const float* __restrict__ X, const uint16_t* __restrict__ W,
                                                  const uint16_t* __restrict__ B, uint16_t* __restrict__ Y, int M,
                                                  int H, float eps) {
@@ -152,7 +158,7 @@ __global__ __launch_bounds__(256) void norm_cast(const float* __restrict__ X, co
     u32x4 g[J], b[J];
     load_f32_row<J>(X + (size_t)row * H, C, lane, lo, hi);
     load_f16_row<J>(W, C, lane, g);
-    if (B) load_f16_row<J>(B, C, lane, b);
+    if constexpr (kBeta) load_f16_row<J>(B, C, lane, b);
     float mean, inv;
     row_stats<J, kLayer>(lo, hi, C, lane, H, eps, mean, inv);
 #pragma unroll
@@ -161,8 +167,8 @@ __global__ __launch_bounds__(256) void norm_cast(const float* __restrict__ X, co
         u32x4 o;
 #pragma unroll
         for (int e = 0; e < 8; e += 2)
-            o[e >> 1] = f32_to_f16_bits(normed<J>(lo, hi, g, b, B != nullptr, j, e, mean, inv)) |
-                        (f32_to_f16_bits(normed<J>(lo, hi, g, b, B != nullptr, j, e + 1, mean, inv)) << 16);
+            o[e >> 1] = f32_to_f16_bits(normed<kBeta>(lo, hi, g, b, j, e, mean, inv)) |
+                        (f32_to_f16_bits(normed<kBeta>(lo, hi, g, b, j, e + 1, mean, inv)) << 16);
         *((u32x4*)(Y + (size_t)row * H) + lane + 64 * j) = o;
     }
 }
@@ -242,14 +248,24 @@ __device__ __forceinline__ void pair_rows(const GemvArgs& a, int p, int& r0, int
     }
 }
 
+// Bound by latency at the benchmark's width: a 3.5 MB product takes 4 us, of which the reads behind one
+// another were the avoidable part. Every read that does not depend on the product goes out at the
+// start; with that and the residual GEMVs' early read of their sum the 12-layer step went from 263 to
+// 255 us per token.
 // Each wave takes NP consecutive row pairs, so the norm of the hidden row (loaded, reduced and
 // formed in every wave) is paid once per 2 NP rows.
-template <int kKind, int J, bool kLayer, int NP>
+// kBeta (a norm bias is given) is a template parameter so that its load goes out with the others: under
+// a branch it came after the row's statistics, one more memory round trip per call.
+template <int kKind, int J, bool kLayer, bool kBeta, int NP>
 __global__ __launch_bounds__(256) void gemv2(GemvArgs a) {
-    const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int unit = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     if (unit >= a.units) return;
     const int K = a.K, C = K / 8;
+    int pos = a.pos;
+    if constexpr (kKind == kQKV) {
+        if (a.pos_dev) pos = *a.pos_dev;
+    }
     int r0[NP], r1[NP];
     u32x4 w0[NP][J], w1[NP][J];
 #pragma unroll
@@ -258,6 +274,7 @@ __global__ __launch_bounds__(256) void gemv2(GemvArgs a) {
         load_f16_row<J, kKind == 2>(a.W + (size_t)r0[p] * K, C, lane, w0[p]);   // lm_head: streamed
         load_f16_row<J, kKind == 2>(a.W + (size_t)r1[p] * K, C, lane, w1[p]);
     }
+    float cs[NP][4];   // kQKV: the rotation's factors
     float y0[NP], y1[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p) y0[p] = y1[p] = 0.f;
@@ -266,7 +283,21 @@ __global__ __launch_bounds__(256) void gemv2(GemvArgs a) {
         u32x4 g[J], b[J];
         load_f32_row<J>(a.x, C, lane, lo, hi);
         load_f16_row<J>(a.gain, C, lane, g);
-        if (a.beta) load_f16_row<J>(a.beta, C, lane, b);
+        if constexpr (kBeta) load_f16_row<J>(a.beta, C, lane, b);
+        // Read here and not after the product, behind which the position and then the factors were
+        // two more memory round trips of every call.
+        if constexpr (kKind == kQKV) {
+            const size_t off = a.pos_dev ? (size_t)pos * a.D : 0;
+            const int half = a.D / 2;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                const float *cr = a.cos_row + off + r0[p] % a.D, *sr = a.sin_row + off + r0[p] % a.D;
+                cs[p][0] = load_early(cr);
+                cs[p][1] = load_early(sr);
+                cs[p][2] = load_early(cr + half);
+                cs[p][3] = load_early(sr + half);
+            }
+        }
         float mean, inv;
         row_stats<J, kLayer>(lo, hi, C, lane, K, a.eps, mean, inv);
 #pragma unroll
@@ -275,7 +306,7 @@ __global__ __launch_bounds__(256) void gemv2(GemvArgs a) {
             if constexpr (kKind == kLogits) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float xe = normed<J>(lo, hi, g, b, a.beta != nullptr, j, e, mean, inv);
+                    const float xe = normed<kBeta>(lo, hi, g, b, j, e, mean, inv);
 #pragma unroll
                     for (int p = 0; p < NP; ++p) {
                         y0[p] = fmaf(half_of(w0[p][j], e), xe, y0[p]);
@@ -286,8 +317,8 @@ __global__ __launch_bounds__(256) void gemv2(GemvArgs a) {
                 u32x4 xn;
 #pragma unroll
                 for (int e = 0; e < 8; e += 2)
-                    xn[e >> 1] = f32_to_f16_bits(normed<J>(lo, hi, g, b, a.beta != nullptr, j, e, mean, inv)) |
-                                 (f32_to_f16_bits(normed<J>(lo, hi, g, b, a.beta != nullptr, j, e + 1, mean, inv))
+                    xn[e >> 1] = f32_to_f16_bits(normed<kBeta>(lo, hi, g, b, j, e, mean, inv)) |
+                                 (f32_to_f16_bits(normed<kBeta>(lo, hi, g, b, j, e + 1, mean, inv))
                                   << 16);
 #pragma unroll
                 for (int p = 0; p < NP; ++p) {
@@ -335,18 +366,10 @@ __global__ __launch_bounds__(256) void gemv2(GemvArgs a) {
                 h1 = f32_to_f16_bits(f16_bits_to_f32(h1) + f16_bits_to_f32(a.bias[rb]));
             }
             const int half = a.D / 2;
-            int pos = a.pos;
-            const float *cos_row = a.cos_row, *sin_row = a.sin_row;
-            if (a.pos_dev) {
-                pos = *a.pos_dev;
-                cos_row += (size_t)pos * a.D;
-                sin_row += (size_t)pos * a.D;
-            }
             if (ra < a.QD + a.KVD) {   // Q or K: rotate the pair (d, d + D/2)
-                const int d = (ra % a.D);
                 const float t0 = f16_bits_to_f32(h0), t1 = f16_bits_to_f32(h1);
-                h0 = f32_to_f16_bits(t0 * cos_row[d] - t1 * sin_row[d]);
-                h1 = f32_to_f16_bits(t1 * cos_row[d + half] + t0 * sin_row[d + half]);
+                h0 = f32_to_f16_bits(t0 * cs[p][0] - t1 * cs[p][1]);
+                h1 = f32_to_f16_bits(t1 * cs[p][2] + t0 * cs[p][3]);
             }
             if (ra < a.QD) {
                 a.q_out[ra] = (uint16_t)h0;
@@ -379,6 +402,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemv_residual_split(const ui
     const int C = K / 8, Q = (C + kSplitWaves - 1) / kSplitWaves;   // chunks per row, per wave
     const int q0 = wave * Q, qn = min(C, q0 + Q) - q0;              // this wave's chunks (qn may be <= 0)
     const int row = blockIdx.x;
+    const float base = load_early(out + row);
     u32x4 w[J], xv[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) {   // loads clamped into the row, masked below
@@ -397,7 +421,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemv_residual_split(const ui
         float acc = part[0];
 #pragma unroll
         for (int i = 1; i < kSplitWaves; ++i) acc += part[i];
-        out[row] += acc;
+        out[row] = base + acc;
     }
 }
 
@@ -454,6 +478,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemv_residual_merge(const fl
     const int C = K / 8, Q = (C + kSplitWaves - 1) / kSplitWaves;
     const int q0 = wave * Q, qn = min(C, q0 + Q) - q0;
     const int row = blockIdx.x;
+    const float base = load_early(out + row);
     u32x4 w[J], xv[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -476,7 +501,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemv_residual_merge(const fl
         float acc = part[0];
 #pragma unroll
         for (int i = 1; i < kSplitWaves; ++i) acc += part[i];
-        out[row] += acc;
+        out[row] = base + acc;
     }
 }
 
@@ -583,10 +608,11 @@ template <int J>
 void norm_cast_launch(bool layer, const float* X, const void* W, const void* B, void* Y, int M, int H, float eps,
                       hipStream_t s) {
     const unsigned grid = ceil_div(M, 4);
-    if (layer)
-        norm_cast<J, true><<<grid, 256, 0, s>>>(X, (const uint16_t*)W, (const uint16_t*)B, (uint16_t*)Y, M, H, eps);
-    else
-        norm_cast<J, false><<<grid, 256, 0, s>>>(X, (const uint16_t*)W, (const uint16_t*)B, (uint16_t*)Y, M, H, eps);
+    const uint16_t *g = (const uint16_t*)W, *b = (const uint16_t*)B;
+    if (layer && b) norm_cast<J, true, true><<<grid, 256, 0, s>>>(X, g, b, (uint16_t*)Y, M, H, eps);
+    else if (layer) norm_cast<J, true, false><<<grid, 256, 0, s>>>(X, g, b, (uint16_t*)Y, M, H, eps);
+    else if (b) norm_cast<J, false, true><<<grid, 256, 0, s>>>(X, g, b, (uint16_t*)Y, M, H, eps);
+    else norm_cast<J, false, false><<<grid, 256, 0, s>>>(X, g, b, (uint16_t*)Y, M, H, eps);
 }
 
 // Row pairs per wave of each kind. The lm_head GEMV (32,000 rows at config 5) has parallelism to
@@ -602,8 +628,10 @@ void gemv_launch(bool layer, GemvArgs a, hipStream_t s) {
     constexpr int NP = pairs_per_wave<kKind>();
     a.units = (a.pairs + NP - 1) / NP;
     const unsigned grid = ceil_div(a.units, 4);
-    if (layer) gemv2<kKind, J, true, NP><<<grid, 256, 0, s>>>(a);
-    else gemv2<kKind, J, false, NP><<<grid, 256, 0, s>>>(a);
+    if (layer && a.beta) gemv2<kKind, J, true, true, NP><<<grid, 256, 0, s>>>(a);
+    else if (layer) gemv2<kKind, J, true, false, NP><<<grid, 256, 0, s>>>(a);
+    else if (a.beta) gemv2<kKind, J, false, true, NP><<<grid, 256, 0, s>>>(a);
+    else gemv2<kKind, J, false, false, NP><<<grid, 256, 0, s>>>(a);
 }
 
 template <int kKind>
