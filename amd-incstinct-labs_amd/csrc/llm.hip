@@ -739,6 +739,24 @@ int llm_logits_argmax(bool layer, const float* hidden, const void* gain, const v
 }
 
 namespace {
+// Copies to host memory: write-through stores, done for the host when the kernel is.
+__global__ __launch_bounds__(256) void copy_f32(const float* __restrict__ src, float* __restrict__ dst, int n) {
+    const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i + 4 <= n) {
+        *(f32x4*)(dst + i) = *(const f32x4*)(src + i);
+    } else {
+        for (int k = i; k < n; ++k) dst[k] = src[k];
+    }
+}
+}  // namespace
+
+// dst[0 .. n) = src, both 16-byte aligned; dst may be pinned host memory.
+int llm_copy_f32(const float* src, float* dst, int n, hipStream_t s) {
+    copy_f32<<<ceil_div(n, 1024), 256, 0, s>>>(src, dst, n);
+    return launch_status();
+}
+
+namespace {
 __global__ void step_state(int* state, int pos, int step) {
     if (threadIdx.x == 0) {
         state[0] = pos;

@@ -59,6 +59,7 @@ int llm_logits_argmax(bool layer, const float* hidden, const void* gain, const v
                       unsigned long long* scratch16, int* ids, int* tokens, int step, hipStream_t s,
                       int* state = nullptr, const void* embed = nullptr, float* next_row = nullptr);
 int llm_step_state(int* state, int pos, int step, hipStream_t s);
+int llm_copy_f32(const float* src, float* dst, int n, hipStream_t s);
 long long attn_decode_plan_key(const cdna3_decode_cfg& c);
 int attn_decode_replayable(const void* q, const void* K, const void* V, void* o, const cdna3_decode_cfg& c, int dtype,
                            void* ws, size_t ws_bytes, const int* len_pos, hipStream_t s);
@@ -175,6 +176,18 @@ struct Session {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     long long gkey = -1;
+    // Logits on their way to a caller that wants every step's: a kernel leaves them in a slot of
+    // pinned host memory and the host copies the slot out while later steps run. (A copy straight
+    // to the caller's memory waits for the step and holds back the next launch: 32 us per step.)
+    // Taken with the first such call; without it (the allocation failed) the copies go straight.
+    static constexpr int kLogitSlots = 4;
+    float* slots = nullptr;
+    hipEvent_t slot_done[kLogitSlots] = {};
+    size_t slot_floats() const { return ((size_t)c.vocab_size + 3) & ~(size_t)3; }
+    bool take_slots();
+    void drop_slots();
+    int put_logits(float* host, int n);
+    int drain_logits(float* host, int n);
 
     int dmalloc(void** p, size_t bytes, bool is_scratch = false) {
         CK(hipMalloc(p, bytes ? bytes : 16));
@@ -484,9 +497,58 @@ int Session::replay_step(int pos) {
     return (int)hipGraphLaunch(gexec, stream);
 }
 
+bool Session::take_slots() {
+    if (slots) return true;
+    if (hipHostMalloc((void**)&slots, kLogitSlots * slot_floats() * 4, hipHostMallocDefault) != hipSuccess) {
+        slots = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    for (hipEvent_t& e : slot_done)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
+            e = nullptr;
+            (void)hipGetLastError();
+            drop_slots();
+            return false;
+        }
+    return true;
+}
+
+void Session::drop_slots() {
+    for (hipEvent_t& e : slot_done) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    if (slots) (void)hipHostFree(slots);
+    slots = nullptr;
+}
+
+// Queues the current logits as row n of host: into slot n % kLogitSlots, whose earlier row is copied
+// out first, or straight there without slots.
+int Session::put_logits(float* host, int n) {
+    const size_t V = c.vocab_size;
+    if (!slots) {
+        CK(hipMemcpyAsync(host + (size_t)n * V, logits, V * 4, hipMemcpyDeviceToHost, stream));
+        return 0;
+    }
+    if (n >= kLogitSlots) CK(drain_logits(host, n - kLogitSlots));
+    const int i = n % kLogitSlots;
+    CK(llm_copy_f32(logits, slots + i * slot_floats(), c.vocab_size, stream));
+    return (int)hipEventRecord(slot_done[i], stream);
+}
+
+int Session::drain_logits(float* host, int n) {
+    const size_t V = c.vocab_size;
+    const int i = n % kLogitSlots;
+    CK(hipEventSynchronize(slot_done[i]));
+    memcpy(host + (size_t)n * V, slots + i * slot_floats(), V * 4);
+    return 0;
+}
+
 void Session::release() {
     if (stream) (void)hipStreamSynchronize(stream);
     drop_graph();
+    drop_slots();
     for (void* ptr : scratch) (void)hipFree(ptr);
     for (void* ptr : allocs) (void)hipFree(ptr);
     scratch.clear();
@@ -568,11 +630,11 @@ extern "C" int cdna3_session_generate(cdna3_session* s, const int* ids, int n_id
     CK(hipEventCreate(&e1));
     CK(hipEventCreate(&e2));
     int rc = 0;
-    const size_t V = S.c.vocab_size;
+    if (step_logits && max_new_tokens > 1) (void)S.take_slots();
     auto body = [&]() -> int {
         CK(hipEventRecord(e0, S.stream));
         CK(S.prefill(ids, n_ids));
-        if (step_logits) CK(hipMemcpyAsync(step_logits, S.logits, V * 4, hipMemcpyDeviceToHost, S.stream));
+        if (step_logits) CK(S.put_logits(step_logits, 0));
         CK(hipEventRecord(e1, S.stream));
         int produced = 1;
         if (S.use_graph && max_new_tokens > 1) CK(llm_step_state(S.dstate, n_ids, 1, S.stream));
@@ -586,11 +648,13 @@ extern "C" int cdna3_session_generate(cdna3_session* s, const int* ids, int n_id
             const int pos = n_ids + step - 1;
             if (S.use_graph) CK(S.replay_step(pos));
             else CK(S.decode_step(pos, step, false));
-            if (step_logits)
-                CK(hipMemcpyAsync(step_logits + (size_t)step * V, S.logits, V * 4, hipMemcpyDeviceToHost, S.stream));
+            if (step_logits) CK(S.put_logits(step_logits, step));
             ++produced;
         }
         CK(hipEventRecord(e2, S.stream));
+        if (step_logits && S.slots)
+            for (int n = std::max(0, produced - Session::kLogitSlots); n < produced; ++n)
+                CK(S.drain_logits(step_logits, n));
         CK(hipMemcpyAsync(out_tokens, S.tokens, (size_t)produced * 4, hipMemcpyDeviceToHost, S.stream));
         CK(hipStreamSynchronize(S.stream));
         *n_out = produced;
