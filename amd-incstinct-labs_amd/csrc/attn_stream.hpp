@@ -55,6 +55,19 @@ __device__ __forceinline__ void wait_copies_younger(int y) {
     }
 }
 
+// The query operands, loaded before the first copies, are waited for behind those: the first chunk and
+// the queries then cost one memory round trip together. (Without a wait here the compiler, which
+// does not know of the copies, would wait for all of them in the loop.) A wait after each of the
+// queries' loads, before the copies, cost decode_wg 5.2 against 4.7 us at D 128 and 118 keys, 26.6
+// against 25.9 at 32 x 8 caches of 1,000, and at D 64 24.6 against 23.4 at 64 x 12 of 500 (a cache
+// of one chunk per wave at D 64 measured the same). decode_mfma keeps its own waits: here the
+// compiler loads its queries in branches and short splits ran 1-2 % slower.
+template <int ND>
+__device__ __forceinline__ void wait_q(const u32x4 (&qb)[1][ND]) {
+#pragma unroll
+    for (int c = 0; c < ND; ++c) asm volatile("" : : "v"(qb[0][c]));
+}
+
 // Copy keys [k0, k0 + kDecT) of one head (row stride rs elements; rows past N re-read key N-1,
 // they are masked) into a ring stage, 16-byte chunks of a row XOR-swizzled as the tile reads expect
 // (the K swizzle when kIsK, else the V swizzle); kNT: non-temporal copies (see dma16).
@@ -105,6 +118,7 @@ __device__ __forceinline__ void stream_keys(const uint16_t* Kh, const uint16_t* 
             load_stage<D, true, kNT>(Kh, rs, kbeg + i * kDecT, N, k_lds + i * kStage, lane);
             load_stage<D, false, kNT>(Vh, rs, kbeg + i * kDecT, N, v_lds + i * kStage, lane);
         }
+    wait_q(qb);
     int st = 0;   // stage of chunk ch
     for (int ch = 0; ch < nch; ++ch) {
         const int ahead = ch + NS - 1;

@@ -80,7 +80,6 @@ __device__ __forceinline__ void load_q(const DecodeArgs& a, int b, int qh0, int 
         qb[0][c] = u32x4{0u, 0u, 0u, 0u};
         if (li < nrows)
             qb[0][c] = *(const u32x4*)((const uint16_t*)a.q + ((size_t)b * a.nQH + qh0 + li) * D + c * 32 + g * 8);
-        asm volatile("" : : "v"(qb[0][c]));   // the loads complete before the first copy is issued
     }
 }
 

@@ -1230,7 +1230,6 @@ __global__ __launch_bounds__(64 * W) void fa_small(PrefillArgs a) {
     for (int c = 0; c < ND; ++c) {
         qb[0][c] = u32x4{0u, 0u, 0u, 0u};
         if (li < nrows) qb[0][c] = *(const u32x4*)(Qh + (q0 + li) * a.q_rs + c * 32 + g * 8);
-        asm volatile("" : : "v"(qb[0][c]));   // the loads complete before the first copy is issued
     }
     const int kend = a.causal ? min(a.seqK, q0 + 16) : a.seqK;
     const int kpw = ((kend + W - 1) / W + stream::kDecT - 1) / stream::kDecT * stream::kDecT;
