@@ -441,6 +441,100 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
+// ---- up to 16 rows of X: K split over the waves of a workgroup ----------------------------------
+// Bound by the read of W in principle, by the chain of K stages in the ring (0.2 us each at 48 of
+// them). Here every workgroup takes all rows of X and 16 output columns (kSilu: 16 gate and 16 up rows
+// of W), wave w the w-th of kRowsWaves parts of K, straight from memory to registers: each W byte is
+// read once and a wave's chain is an eighth. The waves' sums meet in LDS. Measured at M 1 and 16 (us,
+// before: ring): N x K 768 x 3072 11.1 -> 6.1, 11.3 -> 7.6; 4096 x 4096 15.1 -> 10.9, 15.1 -> 13.1;
+// 768 x 768 4.4 -> 3.1, 4.6 -> 3.7; SiLU 768 x 3072 15.9 -> 8.5, 15.8 -> 10.5.
+// Tried and slower: batches of 8 steps' loads ahead of the MFMAs, with the part's last step read
+// again past its end (768 x 768 at M 16: 5.9 against 3.6; a wave's load spans 16 rows of 64 bytes, so
+// loads are what costs); 16 waves (level); 17 to 64 rows (4096 x 4096 at 32 rows: ring 15.1, here 17.4).
+constexpr int kRowsMax = 16, kRowsWaves = 8;
+
+template <int kOut, bool kAccum>
+__global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows(const uint16_t* __restrict__ X,
+                                                             const uint16_t* __restrict__ W, void* __restrict__ Y,
+                                                             int M, int N, int K, int ldy) {
+    constexpr bool kSilu = kOut == kOutSilu;
+    constexpr int NT = kSilu ? 2 : 1;
+    constexpr int kUnroll = 8;
+    __shared__ __attribute__((aligned(16))) gf32x4 part[kRowsWaves][NT][64];
+    const int ncols = kSilu ? N / 2 : N;
+    const int lane = (int)(threadIdx.x & 63u);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int li = lane & 15, g = lane >> 4;
+    const int n0 = (int)blockIdx.x * 16;
+    const int steps = K / 32, per = (steps + kRowsWaves - 1) / kRowsWaves;
+    const int s0 = min(steps, wave * per), s1 = min(steps, s0 + per);
+    const u32x4* wp[NT];   // step s: 16-byte chunk 4 s + g of the row
+#pragma unroll
+    for (int i = 0; i < NT; ++i) wp[i] = (const u32x4*)(W + (size_t)(i * ncols + min(n0 + li, ncols - 1)) * K) + g;
+    const u32x4* xp = (const u32x4*)(X + (size_t)min(li, M - 1) * K) + g;
+    gf32x4 acc[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) acc[i] = gf32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += kUnroll) {
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            if (s + u >= s1) break;
+            const int c = 4 * (s + u);
+            const u32x4 b = xp[c];
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gf16x8, wp[i][c]),
+                                                                __builtin_bit_cast(gf16x8, b), acc[i], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NT; ++i) part[wave][i][lane] = acc[i];
+    __syncthreads();
+    const int n = n0 + 4 * g;
+    if (wave != 0 || li >= M || n >= ncols) return;
+    gf32x4 v = acc[0], t = acc[NT - 1];
+#pragma unroll
+    for (int w = 1; w < kRowsWaves; ++w) {
+        v += part[w][0][lane];
+        if constexpr (kSilu) t += part[w][1][lane];
+    }
+    if constexpr (kSilu) {
+        uint32_t h[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = f32_to_f16_bits(v[e] / (1.f + expf(-v[e])) * t[e]);
+        *(u32x2*)((uint16_t*)Y + (size_t)li * ldy + n) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    } else if constexpr (kOut == kOutF32) {
+        float* y = (float*)Y + (size_t)li * ldy + n;
+        if constexpr (kAccum) v += *(const gf32x4*)y;
+        *(gf32x4*)y = v;
+    } else {
+        _Float16* y = (_Float16*)Y + (size_t)li * ldy + n;
+        if constexpr (kAccum) {
+            const gf16x4 o = *(const gf16x4*)y;
+            v += gf32x4{(float)o[0], (float)o[1], (float)o[2], (float)o[3]};
+        }
+        *(gf16x4*)y = gf16x4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+    }
+}
+
+// Shapes gemm_rows takes: one round of workgroups (8192 x 2048 at M 1 and 16: ring 9.7 and 9.8 us, here
+// 10.0 and 12.6) and a K of four stages (1024 x 256: 2.8 -> 2.3, 2.9 -> 2.5); the tile query's callers
+// rely on the ring below that.
+bool takes_rows(int M, int ncols, int K, int cus) {
+    return M <= kRowsMax && K >= 4 * kBK && (ncols + 15) / 16 <= cus;
+}
+
+int gemm_rows_launch(const uint16_t* X, const uint16_t* W, void* Y, int out, bool accum, int M, int N, int K, int ldy,
+                     hipStream_t s) {
+    const unsigned grid = ceil_div((size_t)(out == kOutSilu ? N / 2 : N), 16), block = 64 * kRowsWaves;
+    if (out == kOutSilu) gemm_rows<kOutSilu, false><<<grid, block, 0, s>>>(X, W, Y, M, N, K, ldy);
+    else if (out == kOutF32 && accum) gemm_rows<kOutF32, true><<<grid, block, 0, s>>>(X, W, Y, M, N, K, ldy);
+    else if (out == kOutF32) gemm_rows<kOutF32, false><<<grid, block, 0, s>>>(X, W, Y, M, N, K, ldy);
+    else if (accum) gemm_rows<kOutF16, true><<<grid, block, 0, s>>>(X, W, Y, M, N, K, ldy);
+    else gemm_rows<kOutF16, false><<<grid, block, 0, s>>>(X, W, Y, M, N, K, ldy);
+    return launch_status();
+}
+
 template <int BM, int BN>
 int gemm_launch(const uint16_t* X, const uint16_t* W, void* Y, bool y_f32, bool accum, int M, int N, int K, int ldy,
                 hipStream_t s) {
@@ -550,6 +644,7 @@ Tile pick_big(int M, int N, int K, int cus, bool silu, const Tile& t) {
 
 // The tile of cdna4_gemm_f16_nt (or, silu, of cdna4_gemm_f16_nt_silu; N counts gate and up rows).
 Tile choose_tile(int M, int N, int K, int cus, bool silu) {
+    if (takes_rows(M, silu ? N / 2 : N, K, cus)) return Tile{kRowsMax, silu ? 32 : 16};
     const Tile t = pick_tile(M, N, K, cus, silu);
     const Tile big = pick_big(M, N, K, cus, silu, t);
     return big.bm ? big : t;
@@ -572,6 +667,7 @@ int llm_gemm_f16(const uint16_t* X, const uint16_t* W, void* Y, bool y_f32, bool
     if (((uintptr_t)X | (uintptr_t)W) % 16 || (uintptr_t)Y % (y_f32 ? 16 : 8)) return -1;
     if ((uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)N * K * 2 >= (1ull << 32)) return -1;   // 32-bit copy offsets
     const int cus = device_cus() > 0 ? device_cus() : 256;
+    if (takes_rows(M, N, K, cus)) return gemm_rows_launch(X, W, Y, y_f32 ? kOutF32 : kOutF16, accum, M, N, K, ldy, s);
     Tile t = choose_tile(M, N, K, cus, false);
     if (cold && t.bm == 32 && t.bn == 32 && M >= 64 &&
         (double)ceil_div((size_t)M, 64) * ceil_div((size_t)N, 32) <= 2.0 * cus)
@@ -630,7 +726,9 @@ int llm_gemm_f16_silu(const uint16_t* X, const uint16_t* W, void* Y, int M, int 
     if (M <= 0 || F <= 0 || K <= 0 || K % kKMul || F % 4 || ldy % 4 || ldy < F) return -1;
     if (((uintptr_t)X | (uintptr_t)W) % 16 || (uintptr_t)Y % 8) return -1;
     if ((uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)2 * F * K * 2 >= (1ull << 32)) return -1;
-    const Tile t = choose_tile(M, 2 * F, K, device_cus() > 0 ? device_cus() : 256, true);
+    const int cus = device_cus() > 0 ? device_cus() : 256;
+    if (takes_rows(M, F, K, cus)) return gemm_rows_launch(X, W, Y, kOutSilu, false, M, 2 * F, K, ldy, s);
+    const Tile t = choose_tile(M, 2 * F, K, cus, true);
 #define CDNA4_GEMM_TILE(a, b) \
     if (t.bm == a && t.bn == b) return gemm_silu_launch<a, b>(X, W, Y, M, F, K, ldy, s);
     CDNA4_GEMM_TILE(64, 64) CDNA4_GEMM_TILE(64, 128) CDNA4_GEMM_TILE(128, 64) CDNA4_GEMM_TILE(128, 128)
