@@ -454,6 +454,51 @@ __device__ Acc look_back(const ScanState& st, size_t tile, Op op) {
     return acc;
 }
 
+// Combined value of all tiles (or groups) before `tile`, on every lane, from their totals alone: lane l
+// reads those of tiles l, l + 64, .., kBelow of them at once, until every one is there. Where all
+// tiles are resident together they publish at about the same time, and this takes one round trip
+// after the slowest instead of a walk behind the prefixes; the order of a float sum is fixed.
+constexpr int kBelow = 8;
+
+template <typename Acc, class Op>
+__device__ __forceinline__ Acc all_below(const ScanState& st, size_t tile, Op op) {
+    const unsigned lane = threadIdx.x;
+    const Acc id = Op::template identity<Acc>();
+    Acc acc = id;
+    for (size_t from = 0; from < tile; from += 64 * kBelow) {
+        Acc a[kBelow];
+        uint32_t waiting = 0;   // slots of this lane not seen yet
+#pragma unroll
+        for (int s = 0; s < kBelow; ++s) {
+            a[s] = id;
+            if (from + lane + 64u * s < tile) waiting |= 1u << s;
+        }
+        for (uint32_t spin = 0;; ++spin) {
+#pragma unroll
+            for (int s = 0; s < kBelow; ++s) {
+                if (waiting & (1u << s)) {
+                    Acc x;
+                    if (read_slot<Acc>(st.agg, (long long)(from + lane + 64u * s), st.tag_agg, x)) {
+                        a[s] = x;
+                        waiting &= ~(1u << s);
+                    }
+                }
+            }
+            if (__ballot(waiting != 0u) == 0ull) break;
+            if (spin >= st.spin_limit) {
+                if (lane == 0) __hip_atomic_store(st.error, st.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        Acc t = a[0];
+#pragma unroll
+        for (int s = 1; s < kBelow; ++s) t = op(t, a[s]);
+        acc = op(acc, allreduce(t, op));
+    }
+    return acc;
+}
+
 // Wave w of workgroup g scans tile g W + w (scan_layout::group_tile, W = scan_waves: 4, or 8 for
 // 8-byte inputs); the group runs one look-back for its W tiles. With one tile per single-wave
 // workgroup the look-back was the bound: per-tile stamps showed a tile's loads arriving after
@@ -463,7 +508,8 @@ __device__ Acc look_back(const ScanState& st, size_t tile, Op op) {
 // 83 us, 64-bit 253 -> 202 us, and 200 -> 187 us with eight-wave groups).
 template <int DT> constexpr int scan_group_waves() { return scan_layout::scan_waves((int)sizeof(typename ScanElem<DT>::In)); }
 
-template <int DT, class Op, bool kVec, int U>
+// kAll: the groups' prefixes from all totals below (all_below) instead of the look-back.
+template <int DT, class Op, bool kVec, int U, bool kAll>
 __device__ __forceinline__ void scan_group(const void* __restrict__ in_, size_t n, void* __restrict__ out_,
                                            const ScanState& st) {
     constexpr int kWaves = scan_group_waves<DT>();
@@ -612,7 +658,11 @@ __device__ __forceinline__ void scan_group(const void* __restrict__ in_, size_t 
     }
     if (wave == 0) {
         Acc gex = id;
-        if (group == 0) {
+        if constexpr (kAll) {
+            publish(st.agg, group, gtot, st.tag_agg);
+            if (group == 0 && lane == 0) *st.epoch_word = st.epoch;
+            gex = all_below<Acc>(st, group, op);
+        } else if (group == 0) {
             publish(st.pre, group, gtot, st.tag_pre);
             if (lane == 0) *st.epoch_word = st.epoch;   // scan status: the workspace's latest call
         } else {
@@ -660,18 +710,22 @@ __device__ __forceinline__ void scan_group(const void* __restrict__ in_, size_t 
     }
 }
 
-// kVec: large tiles of aligned calls; otherwise the small tiles of mid-size calls of any alignment.
+// kVec: large tiles of aligned calls; otherwise the small tiles of mid-size calls of any alignment, whose
+// groups (fewer than 1,024) read all totals below, except of 8-byte inputs, whose groups of eight waves
+// do not all fit the chip (i64 6,000,001, 367 groups: 24.1 us against 21.7). Against the look-back
+// 8,388,608 f32 16.2 -> 13.6 us, f16 13.9 -> 12.2, and a sum's error is that of a tree and not of a
+// chain (5,000,000 f32: 6.4e-8 -> 5.4e-8 relative).
 template <int DT, class Op, bool kVec>
 __global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_tiles(const void* __restrict__ in_, size_t n,
                                                                           void* __restrict__ out_, ScanState st) {
-    scan_group<DT, Op, kVec, scan_u<DT, kVec>()>(in_, n, out_, st);
+    scan_group<DT, Op, kVec, scan_u<DT, kVec>(), !kVec && sizeof(typename Elem<DT>::In) != 8>(in_, n, out_, st);
 }
 
 // Large tiles of misaligned calls (small ones measured 111, 98 and 202 us at 2^26: f32, f16, i64).
 template <int DT, class Op>
 __global__ __launch_bounds__(64 * scan_group_waves<DT>()) void scan_wide(const void* __restrict__ in_, size_t n,
                                                                          void* __restrict__ out_, ScanState st) {
-    scan_group<DT, Op, false, scan_u<DT, true>()>(in_, n, out_, st);
+    scan_group<DT, Op, false, scan_u<DT, true>(), false>(in_, n, out_, st);
 }
 
 // The last n % VEC (< VEC) elements of an aligned call, after scan_tiles has published every
@@ -702,12 +756,9 @@ __global__ __launch_bounds__(64) void scan_tail(const void* __restrict__ in_, si
 // Bound by launch and latency: a load, a store and one round trip through the slots. Up to
 // kSpreadTiles tiles of 64 x U vectors, one wave and workgroup each, so that a mid-size input
 // reaches every CU (groups of 32,768 fp32 elements leave a million on 31 of them) and a small one is
-// done by a few short waves. All tiles are resident together and publish their totals at about the
-// same time, so a tile does not walk back window by window: lane l of its wave reads the totals of
-// tiles l, l + 64, .. below it, all loads issued at once, until every one is there: one round trip
-// after the slowest. Vectors lie at any element; the last tile's elements go one by one (no tail
+// done by a few short waves. A tile's prefix comes from all totals below it (all_below). Vectors lie at any element; the last tile's elements go one by one (no tail
 // launch). Sizes and times: scan_layout::spread_u.
-using scan_layout::kSpreadTiles;
+static_assert(scan_layout::kSpreadTiles <= 64 * kBelow, "one pass of all_below");
 
 template <int DT, class Op, int U>
 __global__ __launch_bounds__(64) void scan_spread(const void* __restrict__ in_, size_t n, void* __restrict__ out_,
@@ -757,37 +808,7 @@ __global__ __launch_bounds__(64) void scan_spread(const void* __restrict__ in_, 
     if (gridDim.x > 1) publish(st.agg, tile, run, st.tag_agg);
     if (tile == 0 && lane == 0) *st.epoch_word = st.epoch;   // scan status: the workspace's latest call
     Acc excl = id;
-    if (tile > 0) {
-        constexpr int S = kSpreadTiles / 64;
-        Acc a[S];
-        uint32_t waiting = 0;   // slots of this lane not seen yet
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            a[s] = id;
-            if (lane + 64u * s < tile) waiting |= 1u << s;
-        }
-        for (uint32_t spin = 0;; ++spin) {
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                if (waiting & (1u << s)) {
-                    Acc x;
-                    if (read_slot<Acc>(st.agg, (long long)(lane + 64u * s), st.tag_agg, x)) {
-                        a[s] = x;
-                        waiting &= ~(1u << s);
-                    }
-                }
-            }
-            if (__ballot(waiting != 0u) == 0ull) break;
-            if (spin >= st.spin_limit) {
-                if (lane == 0) __hip_atomic_store(st.error, st.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-#pragma unroll
-        for (int s = 0; s < S; ++s) excl = op(excl, a[s]);
-        excl = allreduce(excl, op);
-    }
+    if (tile > 0) excl = all_below<Acc>(st, tile, op);
     if (full) {
         constexpr int kWords = (int)(sizeof(Out) * VEC / 16);
         u32x4_a4* dst = (u32x4_a4*)tout + lane * kWords;

@@ -84,10 +84,10 @@ constexpr int spread_u(size_t n, int VEC) {
 }
 // Above that large tiles from large_groups groups of them on, one and a half per CU, for 16-bit
 // inputs, whose small tiles are a quarter, one; small tiles below. Fewer groups leave CUs idle
-// (4,194,304 elements: 12.8 -> 10.9, 17.0 -> 9.7, 19.2 -> 14.9; 8,388,608: 17.7 -> 16.3, 18.2 ->
-// 13.9, 25.2 -> 25.4), more have fewer look-backs in large tiles (16,777,216: small 27.5, 24.3,
-// 51.0, large 25.8, 20.4, 48.0; just below the line, 12,000,000: small 21.2, 18.6, 38.3, large 21.4,
-// 19.1, 42.2).
+// (4,194,304 elements: 12.8 -> 10.2, 17.0 -> 9.1, 19.2 -> 14.9; 8,388,608: 17.7 -> 13.6, 18.2 ->
+// 12.2, 25.2 -> 25.7; 12,000,000: 21.4 -> 18.8, 19.1 -> 16.1, 42.2 -> 38.3), more have fewer prefixes
+// to wait for in large tiles (16,777,216 with the look-back in both: small 27.5, 24.3, 51.0, large
+// 25.8, 20.4, 48.0).
 constexpr int large_groups(int in_bytes) { return in_bytes == 2 ? 256 : 384; }
 constexpr bool large_tiles(size_t n, int VEC, int in_bytes) {
     return groups_for(tiles_for(n, VEC, scan_u(in_bytes, true)), scan_waves(in_bytes)) >= (size_t)large_groups(in_bytes);
