@@ -27,14 +27,15 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float f) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f);
 }
 
-// Rotate-half RoPE of one (d, d + D/2) pair of fp16 values with the pair's cos/sin entries
-// (shared by the fused RoPE + append kernel and the prompt GEMM's Q|K|V epilogue, so both round
-// alike).
+// Rotate-half RoPE of one (d, d + D/2) pair of fp16 values with the pair's cos/sin entries, shared by
+// every kernel that writes the cache (the RoPE + append kernel, the prompt GEMM's Q|K|V epilogue, the
+// decode step's GEMV): the fused multiply-adds are written out, since left to contraction the
+// product that is rounded by itself differed from kernel to kernel, and with it a few cache rows.
 __device__ __forceinline__ void rope_pair(uint32_t a_bits, uint32_t b_bits, float c_lo, float s_lo, float c_hi,
                                           float s_hi, uint32_t& lo, uint32_t& hi) {
     const float a = f16_bits_to_f32(a_bits), b = f16_bits_to_f32(b_bits);
-    lo = f32_to_f16_bits(a * c_lo + (-b) * s_lo);
-    hi = f32_to_f16_bits(b * c_hi + a * s_hi);
+    lo = f32_to_f16_bits(fmaf(c_lo, a, -(b * s_lo)));
+    hi = f32_to_f16_bits(fmaf(c_hi, b, a * s_hi));
 }
 
 // Destinations of the prompt GEMM's Q|K|V epilogue (gemm.hip, llm_gemm_qkv_rope): queries

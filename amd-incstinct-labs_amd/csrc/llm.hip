@@ -366,11 +366,8 @@ __global__ __launch_bounds__(256) void gemv2(GemvArgs a) {
                 h1 = f32_to_f16_bits(f16_bits_to_f32(h1) + f16_bits_to_f32(a.bias[rb]));
             }
             const int half = a.D / 2;
-            if (ra < a.QD + a.KVD) {   // Q or K: rotate the pair (d, d + D/2)
-                const float t0 = f16_bits_to_f32(h0), t1 = f16_bits_to_f32(h1);
-                h0 = f32_to_f16_bits(t0 * cs[p][0] - t1 * cs[p][1]);
-                h1 = f32_to_f16_bits(t1 * cs[p][2] + t0 * cs[p][3]);
-            }
+            if (ra < a.QD + a.KVD)   // Q or K: rotate the pair (d, d + D/2)
+                rope_pair(h0, h1, cs[p][0], cs[p][1], cs[p][2], cs[p][3], h0, h1);
             if (ra < a.QD) {
                 a.q_out[ra] = (uint16_t)h0;
                 a.q_out[rb] = (uint16_t)h1;

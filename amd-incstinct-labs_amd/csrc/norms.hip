@@ -322,12 +322,10 @@ __global__ __launch_bounds__(256) void rope_pairs(uint16_t* __restrict__ T, cons
     uint16_t* t = T + sh * D;
     const float* c = cosv + (size_t)s * D;
     const float* sn = sinv + (size_t)s * D;
-    const float a = f16_bits_to_f32(t[d]);
-    const float b = f16_bits_to_f32(t[d + half]);
-    const float lo = a * c[d] + (-b) * sn[d];
-    const float hi = b * c[d + half] + a * sn[d + half];
-    t[d] = (uint16_t)f32_to_f16_bits(lo);
-    t[d + half] = (uint16_t)f32_to_f16_bits(hi);
+    uint32_t lo, hi;
+    rope_pair(t[d], t[d + half], c[d], sn[d], c[d + half], sn[d + half], lo, hi);
+    t[d] = (uint16_t)lo;
+    t[d + half] = (uint16_t)hi;
 }
 
 __global__ __launch_bounds__(256) void rope_table(float* __restrict__ cosv, float* __restrict__ sinv, int pos0,
