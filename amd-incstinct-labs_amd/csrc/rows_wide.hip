@@ -65,6 +65,20 @@ __device__ __forceinline__ float row_combine(float v, Op op, float* slot) {
     return v;
 }
 
+// A vector's own elements (those from sk on; 0 in the place of the others) less `mean`.
+__device__ __forceinline__ f32x4 own(f32x4 v, int sk, float mean = 0.f) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = e >= sk ? v[e] - mean : 0.f;
+    return v;
+}
+// Sums of a vector, in pairs as in the wave-per-row kernels, whose results unaligned rows of one wave then
+// give bit for bit. Error against 64 bits, softmax: in sequence 6.5e-8 at 2,047 columns, 5.9e-8 at 5,000,
+// in pairs 5.6e-8 and 5.4e-8 (element-wise kernels 6.1e-8, 7.4e-8). Rows a little wider than 64 or 128
+// keep 2-6 % more than the element-wise kernels (67: 6.4e-8 -> 6.7e-8): their last vector is alone in
+// its 16 lanes, one more addition at the row's full size.
+__device__ __forceinline__ float sum4(f32x4 v) { return (v[0] + v[1]) + (v[2] + v[3]); }
+__device__ __forceinline__ float sumsq4(f32x4 v) { return (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); }
+
 constexpr int kBlock = 256;
 
 // One row per TPR threads: workgroups of 256 threads (TPR 64: four rows each; 256: one), or of 1,024.
@@ -96,12 +110,9 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rows_kernel(const
         float s = 0.f;
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const int sk = skip(k);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[k][e] = __expf(v[k][e] - m);
-                s += e >= sk ? v[k][e] : 0.f;
-            }
+            for (int e = 0; e < 4; ++e) v[k][e] = __expf(v[k][e] - m);
+            s += sum4(own(v[k], skip(k)));
         }
         const float inv = 1.f / row_combine<TPR>(s, Sum{}, slots[1]);
 #pragma unroll
@@ -114,23 +125,13 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rows_kernel(const
         if constexpr (kOp == kRowsLayer) {
             float s = 0.f;
 #pragma unroll
-            for (int k = 0; k < NV; ++k) {
-                const int sk = skip(k);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s += e >= sk ? v[k][e] : 0.f;
-            }
+            for (int k = 0; k < NV; ++k) s += sum4(own(v[k], skip(k)));
             mean = row_combine<TPR>(s, Sum{}, slots[0]) / (float)H;
         }
         float q = 0.f;
 #pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const int sk = skip(k);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float d = v[k][e] - mean;
-                q += e >= sk ? d * d : 0.f;
-            }
-        }
+        for (int k = 0; k < NV; ++k)
+            q += sumsq4(own(v[k], skip(k), mean));
         const float inv = rsqrtf(row_combine<TPR>(q, Sum{}, slots[1]) / (float)H + eps);
 #pragma unroll
         for (int k = 0; k < NV; ++k) {

@@ -63,3 +63,16 @@ def test_softmax_masked_rows(H):
     want /= want.sum(axis=1, keepdims=True)
     np.testing.assert_allclose(got[:3], want, rtol=1e-5, atol=1e-37)
     assert np.isnan(got[3]).all()
+
+
+@pytest.mark.parametrize("M,H", [(1100, 260), (1100, 1024), (1030, 2048)])
+def test_rows_at_any_element_equal_aligned_rows(M, H):
+    # One wave per row in both cases, the same columns per lane and the same order of the sums: the
+    # start of the rows may not change a bit (M above the line of few rows).
+    x = torch.from_numpy(oracle.normal(M + H, M * H, 0.0, 2.0)).to(DEV)
+    g, b = torch.from_numpy(oracle.uniform(1, H, 0.5, 1.5)).to(DEV), torch.from_numpy(oracle.uniform(2, H)).to(DEV)
+    buf = torch.empty(M * H + 1, device=DEV)
+    buf[1:] = x
+    X, U = x.reshape(M, H), buf[1:].reshape(M, H)
+    assert torch.equal(cdna4.softmax_rows_f32(U), cdna4.softmax_rows_f32(X))
+    assert torch.equal(cdna4.layernorm_f32(U, g, b, 1e-5), cdna4.layernorm_f32(X, g, b, 1e-5))
