@@ -85,12 +85,19 @@ constexpr int spread_u(size_t n, int VEC) {
 // Above that large tiles from large_groups groups of them on, one and a half per CU, for 16-bit
 // inputs, whose small tiles are a quarter, one; small tiles below. Fewer groups leave CUs idle
 // (4,194,304 elements: 12.8 -> 10.2, 17.0 -> 9.1, 19.2 -> 14.9; 8,388,608: 17.7 -> 13.6, 18.2 ->
-// 12.2, 25.2 -> 25.7; 12,000,000: 21.4 -> 18.8, 19.1 -> 16.1, 42.2 -> 38.3), more have fewer prefixes
+// 12.2, 23.0 -> 22.8; 12,000,000: 21.4 -> 18.8, 19.1 -> 16.1, 42.2 -> 38.3), more have fewer prefixes
 // to wait for in large tiles (16,777,216 with the look-back in both: small 27.5, 24.3, 51.0, large
 // 25.8, 20.4, 48.0).
 constexpr int large_groups(int in_bytes) { return in_bytes == 2 ? 256 : 384; }
+// 8-byte inputs also take them where small tiles need more than one group per CU and large ones do not
+// (4.2 to 8.4 million elements): their groups are eight waves, and a second round of them waits for
+// the first. Small / large, i64: 5,000,012 elements 19.4 / 18.2, 6,291,456 21.4 / 19.3, 8,388,608 24.7 /
+// 22.8; vectors at odd elements 19.4 / 19.7, 21.9 / 20.6, 26.2 / 26.6.
+constexpr size_t kOneRound = 256;
 constexpr bool large_tiles(size_t n, int VEC, int in_bytes) {
-    return groups_for(tiles_for(n, VEC, scan_u(in_bytes, true)), scan_waves(in_bytes)) >= (size_t)large_groups(in_bytes);
+    const size_t large = groups_for(tiles_for(n, VEC, scan_u(in_bytes, true)), scan_waves(in_bytes));
+    const size_t small = groups_for(tiles_for(n, VEC, scan_u(in_bytes, false)), scan_waves(in_bytes));
+    return large >= (size_t)large_groups(in_bytes) || (in_bytes == 8 && large <= kOneRound && small > kOneRound);
 }
 
 // 64-bit word w of group (slot) t's slot (NW words per slot).

@@ -35,6 +35,11 @@ int main(int argc, char** argv) {
                 CHECK(!sl::large_tiles(n, T.VEC, T.in_bytes), "the forms do not overlap");
                 continue;
             }
+            if (T.in_bytes == 8) {   // one round of large groups and not two of small ones (256 CUs)
+                const size_t small_g = sl::groups_for(sl::tiles_for(n, T.VEC, sl::scan_u(8, false)), sl::scan_waves(8));
+                const size_t large_g = sl::groups_for(sl::tiles_for(n, T.VEC, sl::scan_u(8, true)), sl::scan_waves(8));
+                CHECK(small_g <= 256 || large_g > 256 || sl::large_tiles(n, T.VEC, 8), "one round of groups");
+            }
             for (int vec = 0; vec < 2; ++vec) {
                 const bool large = sl::large_tiles(n, T.VEC, T.in_bytes), v = vec && large;
                 const int U = sl::scan_u(T.in_bytes, large), waves = sl::scan_waves(T.in_bytes);

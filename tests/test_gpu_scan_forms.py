@@ -30,6 +30,8 @@ def sizes(dtype):
     out = []
     for u, tiles in ((2, 256), (4, 256), (8, 512), (16, 512)):          # the last size of each single-wave form
         out += [64 * vec * u * tiles + d for d in (-vec - 1, 0, 1)]
+    if dtype.itemsize == 8:   # the large tiles' range of one round of groups
+        out += [group * t + d for t in (128, 256) for d in (-1, 0, 1)]
     return out + [64 * vec * 16 * 1000 + 5, group * (line - 1) - 1, group * (line - 1), group * (line - 1) + 1,
                   group * (line + 7) + vec + 1]
 
