@@ -58,14 +58,17 @@ __device__ __forceinline__ void wait_copies_younger(int y) {
 // The query operands, loaded before the first copies, are waited for behind those: the first chunk and
 // the queries then cost one memory round trip together. (Without a wait here the compiler, which
 // does not know of the copies, would wait for all of them in the loop.) A wait after each of the
-// queries' loads, before the copies, cost decode_wg 5.2 against 4.7 us at D 128 and 118 keys, 26.6
-// against 25.9 at 32 x 8 caches of 1,000, and at D 64 24.6 against 23.4 at 64 x 12 of 500 (a cache
-// of one chunk per wave at D 64 measured the same). decode_mfma keeps its own waits: here the
-// compiler loads its queries in branches and short splits ran 1-2 % slower.
+// queries' loads, before the copies, cost decode_wg 5.0 against 4.5 us at D 128 and 118 keys, 13.6
+// against 13.2 at 16 x 8 caches of 1,000, and at D 64 24.6 against 23.4 at 64 x 12 of 500 (a cache
+// of one chunk per wave at D 64 measured the same). One statement for all operands: with one each
+// the loop of the bf16 kernel at D 128 came out in an order that took 106.7 us for 32 x 8 heads and
+// 16,001 keys where this takes 102.5 and the waits before the copies 103.4. decode_mfma keeps its
+// own waits: here the compiler loads its queries in branches and short splits ran 1-2 % slower.
 template <int ND>
 __device__ __forceinline__ void wait_q(const u32x4 (&qb)[1][ND]) {
-#pragma unroll
-    for (int c = 0; c < ND; ++c) asm volatile("" : : "v"(qb[0][c]));
+    static_assert(ND == 2 || ND == 4, "D = 64 or 128");
+    if constexpr (ND == 4) asm volatile("" : : "v"(qb[0][0]), "v"(qb[0][1]), "v"(qb[0][2]), "v"(qb[0][3]));
+    else asm volatile("" : : "v"(qb[0][0]), "v"(qb[0][1]));
 }
 
 // Copy keys [k0, k0 + kDecT) of one head (row stride rs elements; rows past N re-read key N-1,
