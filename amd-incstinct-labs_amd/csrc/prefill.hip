@@ -1230,6 +1230,10 @@ __global__ __launch_bounds__(64 * W) void fa_small(PrefillArgs a) {
     for (int c = 0; c < ND; ++c) {
         qb[0][c] = u32x4{0u, 0u, 0u, 0u};
         if (li < nrows) qb[0][c] = *(const u32x4*)(Qh + (q0 + li) * a.q_rs + c * 32 + g * 8);
+        // D = 64 has two loads of the queries, and waiting for each before the first copy is the faster order
+        // (wait_q in stream_keys then finds nothing to wait for): B1 H1 S 257 causal f16 4.87 us against
+        // 5.05, H8 S 512 6.04 / 6.18, B3 H17 S 100 5.34 / 5.52.
+        if constexpr (D == 64) asm volatile("" : : "v"(qb[0][c]));
     }
     const int kend = a.causal ? min(a.seqK, q0 + 16) : a.seqK;
     const int kpw = ((kend + W - 1) / W + stream::kDecT - 1) / stream::kDecT * stream::kDecT;
