@@ -125,8 +125,8 @@ __global__ __launch_bounds__(256) void rmsnorm_row16(const float* __restrict__ X
     }
 }
 
-// Rows of fewer than 4 or more than 65,536 columns that the other forms do not take: two passes over
-// the row (the second pass hits the cache).
+// Rows that the other forms do not take (fewer than 4 or more than 65,536 columns, more rows than
+// rows_wide's grid can have): two passes over the row (the second pass hits the cache).
 __global__ __launch_bounds__(256) void rmsnorm_any(const float* __restrict__ X, const uint16_t* __restrict__ W,
                                                    float* __restrict__ Y, int M, int H, float eps) {
     const unsigned lane = threadIdx.x & 63u;

@@ -18,6 +18,7 @@
 // addresses), and the last vector of a row whose width is no multiple of 4 is moved back to end at
 // the row's end: its first `skip` elements then repeat its neighbour's, take no part in the row's
 // sums, and are stored twice with the same value.
+#include "common.hpp"
 #include "rows_wide.hpp"
 #include "wave_primitives/detail/xlane.hpp"
 
