@@ -6,8 +6,8 @@
 // mask "key > query -> excluded", fp32 softmax and accumulation, O / l with an l > 0 guard.
 //
 // MI355X design of the f16 / bf16 kernels (fa_pipe for large problems, fa_mfma_keys below that, with
-// the keys of a query block split over the waves, fa_small for the smallest; fa_mfma for many short
-// causal sequences at D = 64; plan_mfma estimates each and takes the least):
+// the keys of a query block split over the waves, fa_mfma for many short sequences, fa_small for the
+// smallest problems; plan_mfma estimates each and takes the least):
 //   * S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_16x16x32_{f16,bf16}. In that orientation
 //     the S^T accumulator of a lane holds one query column (q = lane % 16) and 4 keys, so
 //     the softmax state (m, l) and the O^T accumulator of a query live in the same lanes:
@@ -1276,29 +1276,42 @@ __global__ __launch_bounds__(64 * W) void fa_small(PrefillArgs a) {
 
 // ---- kernel choice for the 16-bit path ---------------------------------------------------------
 // Five forms cover the range from a few rows to whole batches of long sequences; which is fastest
-// depends on how the items fill the CUs, so each is estimated and the least taken. An item of a form
-// costs `fixed` plus its steps times `step` (us, with the chip nearly idle), and `step` grows by up to
-// `load` as the work fills the chip (the clock falls with the power). The time is the larger of the
-// heaviest item and the CUs' share of all items (plus part of an item where they do not come out
-// even); fa_pipe's persistent workgroups are added up as they run. Constants fitted to sweeps of every
-// form (D 64 and 128, fp16 and bf16, causal and not, 1-64 heads x 1-8 batches, 32-8,192 queries and
-// keys): the pick was the fastest form measured, or within 5 % of it, at all but a few points. E.g.
-// (us, head-on) B1 32/8 heads S 1,531 D 128 causal: fa_mfma_keys<2> 33.5, <4> 40.6, fa_pipe 41.2, the
-// four-wave kernel 50.7; S 512: <4> 12.1, <2> 15.8, fa_pipe 19.7, fa_small 25.1; B1 H12 S 512 D 64:
-// <8> 7.4, <4> 8.2, fa_small 9.1; B1 H8 S 512 D 128: fa_small 9.2, <4> 10.9.
+// depends on how the items fill the CUs, so each is estimated and the least taken. Times in us: an
+// item costs `fixed` (`lo` more in bf16, whose first keys are multiplied twice) plus its steps times
+// `step`, and `step` grows by up to `load` as the work fills the chip (the clock falls with the
+// power). The time is the larger of the heaviest item and the CUs' share of all items, plus `tail` of
+// a mean item where they are more than a round. Where two workgroups share a CU, a step costs
+// `share` in the CUs' share and `pair` in the heaviest item; fa_mfma's order with batch x heads a multiple
+// of 8 (head by head on an XCD, not heaviest first) leaves the longer tail `tail8`. fa_pipe's persistent
+// workgroups are added up as they run; `tail` there is what a later item of a workgroup costs of
+// `fixed`. The constants are fitted to sweeps of every form, the last over 8,500 shapes (D 64 and 128, fp16 and bf16,
+// causal and not, 1-64 heads x 1-64 batches, 1-8,192 queries and keys); what the pick loses against the
+// fastest form, there and at shapes it was not fitted to: profiles/prefill_forms.md. E.g. B1 32/8 heads
+// S 1,531 D 128 causal: fa_mfma_keys<2> 33.5, <4> 40.6, fa_pipe 41.2, fa_mfma 50.7; B3 64/16 S 144 D
+// 128: fa_mfma 11.8, fa_mfma_keys<2> 18.3; B1 H12 S 512 D 64: <8> 7.4, <4> 8.2, fa_small 9.1; B1 H8 S 512
+// D 128: fa_small 9.2, <4> 10.9.
 enum PrefillForm { kFormPipe, kFormKeys2, kFormKeys4, kFormKeys8, kFormMfma4, kFormSmallL, kFormSmallS, kForms };
-struct FormCost { int rows, keys; double fixed, step, load; };   // queries per item, keys per step
+struct FormCost {
+    int rows, keys;   // queries per item, keys per step
+    double fixed, lo, step, load, tail, share, tail8, pair;
+};
 template <int D>
 constexpr FormCost form_cost(int f) {
     constexpr bool d64 = D == 64;
     switch (f) {
-        case kFormPipe: return d64 ? FormCost{256, 64, 4.5, 0.92, 0.22} : FormCost{256, 64, 5.5, 1.36, 0.28};
-        case kFormKeys2: return d64 ? FormCost{128, 64, 4.3, 0.50, 0.30} : FormCost{128, 64, 6.0, 0.70, 0.38};
-        case kFormKeys4: return d64 ? FormCost{64, 128, 3.4, 0.62, 0.15} : FormCost{64, 128, 5.0, 0.95, 0.15};
-        case kFormKeys8: return FormCost{32, 256, 2.8, 0.85, 0.10};      // D = 64 only
-        case kFormMfma4: return FormCost{64, 64, 2.5, 0.67, 0.00};       // D = 64 only
-        case kFormSmallL: return d64 ? FormCost{16, 256, 2.3, 0.66, 0.10} : FormCost{16, 128, 3.4, 0.90, 0.10};
-        default: return d64 ? FormCost{16, 128, 2.5, 1.10, 0.10} : FormCost{16, 64, 3.4, 1.00, 0.00};
+        case kFormPipe: return d64 ? FormCost{256, 64, 4.5, 0, 0.92, 0.22, 0.6, 1, 0, 1}
+                                   : FormCost{256, 64, 4.92, 0, 1.36, 0.27, 0.5, 1, 0, 1};
+        case kFormKeys2: return d64 ? FormCost{128, 64, 4.3, 0, 0.5, 0.3, 0.4, 1, 0.4, 1}
+                                    : FormCost{128, 64, 6, 0, 0.7, 0.37, 0.4, 1, 0.4, 1};
+        case kFormKeys4: return d64 ? FormCost{64, 128, 3.4, 0, 0.62, 0.15, 0.4, 1, 0.4, 1}
+                                    : FormCost{64, 128, 5, 0.14, 0.904, 0.2, 0.41, 1, 0.41, 1};
+        case kFormKeys8: return FormCost{32, 256, 3.43, 0, 0.851, 0.08, 0.3, 1, 0.3, 1};   // D = 64 only
+        case kFormMfma4: return d64 ? FormCost{64, 64, 2.5, 0, 0.67, 0, 0.15, 1.5, 0.15, 1}
+                                    : FormCost{64, 64, 3.34, 0.11, 0.951, 0.2, 0.25, 1.53, 0.54, 1.14};
+        case kFormSmallL: return d64 ? FormCost{16, 256, 2.3, 0, 0.66, 0.1, 0, 1, 0, 1}
+                                     : FormCost{16, 128, 3.4, 0, 0.9, 0.1, 0, 1, 0, 1};
+        default: return d64 ? FormCost{16, 128, 2.31, 0.19, 0.954, 0.09, 0.59, 1, 0.59, 0.97}
+                            : FormCost{16, 64, 3.55, 0.07, 1.098, 0.01, 0.33, 1, 0.33, 0.85};
     }
 }
 
@@ -1328,7 +1341,7 @@ double pipe_load(const cdna3_prefill_cfg& c, const FormCost& fc, double step, in
         for (int item = p; item < items; item += grid) {
             int bh, qrev;
             persistent_item(item, grid, nqb, nbh, order, bh, qrev);
-            t += fc.fixed * (item == p ? 1.0 : 0.6) + step * (double)block_steps(c, fc.rows, fc.keys, nqb - 1 - qrev);
+            t += fc.fixed * (item == p ? 1.0 : fc.tail) + step * (double)block_steps(c, fc.rows, fc.keys, nqb - 1 - qrev);
         }
         worst = std::max(worst, t);
     }
@@ -1339,19 +1352,25 @@ constexpr long long kPipeSimItems = 1 << 15;       // larger grids: many rounds,
 constexpr double kPipeL2Bytes = 4.0 * 1024 * 1024; // an XCD's L2
 
 template <int D>
-PrefillPlan plan_mfma(const cdna3_prefill_cfg& c) {
+PrefillPlan plan_mfma(const cdna3_prefill_cfg& c, bool bf16) {
     const long long heads = (long long)c.batch * c.nQHeads;
     const int cus = device_cus();
     const long long blocks8 = heads * ((c.seqQ + 255) / 256);
     PrefillPlan best{};
     double best_t = 1e300;
     for (int f = 0; f < kForms; ++f) {
-        if ((f == kFormKeys8 || f == kFormMfma4) && D != 64) continue;
-        if (f == kFormMfma4 && !c.causal) continue;
+        if (f == kFormKeys8 && D != 64) continue;
+        // fa_mfma rounds its weights against one maximum per 64 keys where fa_small has one per wave and 32
+        // keys, and lies 2-4 % further from 64 bits in fp16 (fa_pipe lies as far): it serves causal problems
+        // that fa_small does not fit in a round, at D = 128 those of whole rounds only
+        if (f == kFormMfma4 && (!c.causal || (blocks8 < cus && heads * ((c.seqQ + 63) / 64) < 2LL * cus &&
+                                              (D == 128 || heads * ((c.seqQ + 15) / 16) <= cus))))
+            continue;
         // fa_pipe gives the first keys their second bf16 term only where few keys are seen; below whole
         // rounds (a quarter of one non-causal) the other forms, which always do, are as fast
         if (f == kFormPipe && blocks8 < (c.causal ? cus : cus / 4)) continue;
-        const FormCost fc = form_cost<D>(f);
+        FormCost fc = form_cost<D>(f);
+        if (bf16) fc.fixed += fc.lo;
         const long long nqb = (c.seqQ + fc.rows - 1) / fc.rows, items = heads * nqb;
         if (f == kFormSmallL && items > cus) continue;
         if (f == kFormSmallS && items <= cus) continue;
@@ -1373,7 +1392,7 @@ PrefillPlan plan_mfma(const cdna3_prefill_cfg& c) {
             const int pcus = cus & ~7;
             if (pcus >= 8 && p.grid > pcus) p.grid = pcus;
             p.order = heads % 8 == 0 && p.grid % 8 == 0 ? 1 : 0;
-            t = std::max(fc.fixed + step * heavy, (0.6 * fc.fixed * items + step * steps) / p.grid);
+            t = std::max(fc.fixed + step * heavy, (fc.tail * fc.fixed * items + step * steps) / p.grid);
             if (items > p.grid && items <= kPipeSimItems) {
                 t = pipe_load(c, fc, step, (int)p.grid, (int)nqb, (int)heads, p.order);
                 if (p.order == 1 && c.causal) {
@@ -1388,11 +1407,11 @@ PrefillPlan plan_mfma(const cdna3_prefill_cfg& c) {
                 }
             }
         } else {
-            // two fa_mfma workgroups of a CU slow each other's steps by half
-            t = (fc.fixed * items + step * (f == kFormMfma4 ? 1.5 : 1.0) * steps) / slots;
-            if (items > slots) t += (f == kFormMfma4 ? 0.15 : 0.4) * (fc.fixed + step * steps / items);
+            t = (fc.fixed * items + step * fc.share * steps) / slots;
+            if (items > slots)
+                t += (f == kFormMfma4 && heads % 8 == 0 ? fc.tail8 : fc.tail) * (fc.fixed + step * steps / items);
             const double rounds = (f == kFormSmallL || f == kFormSmallS || c.causal) ? 1.0 : (double)((items + slots - 1) / slots);
-            t = std::max(t, rounds * (fc.fixed + step * heavy));
+            t = std::max(t, rounds * (fc.fixed + step * heavy * (slots > cus && items > cus ? fc.pair : 1.0)));
         }
         if (t < best_t) {
             best_t = t;
@@ -1427,7 +1446,7 @@ PrefillArgs make_args(const cdna3_prefill_cfg& c, const cdna3_prefill_strides& s
 template <int D, bool kBf16>
 int dispatch_mfma(const cdna3_prefill_cfg& c, const cdna3_prefill_strides& st, const void* Q, const void* K,
                   const void* V, void* O, hipStream_t s) {
-    const PrefillPlan p = plan_mfma<D>(c);
+    const PrefillPlan p = plan_mfma<D>(c, kBf16);
     const long long nbh = (long long)c.batch * c.nQHeads;
     if (p.rows == 0) return CDNA4_ERR_INVALID_VALUE;   // more items than a grid holds
     PrefillArgs a = make_args(c, st, Q, K, V, O, p.rows);
@@ -1441,11 +1460,10 @@ int dispatch_mfma(const cdna3_prefill_cfg& c, const cdna3_prefill_strides& st, c
         case kFormKeys4: fa_mfma_keys<D, 4, 1, kBf16><<<grid, 512, 0, s>>>(a); break;
         case kFormSmallL: fa_small<D, kBf16, small_waves<D>(true)><<<grid, 64 * small_waves<D>(true), 0, s>>>(a); break;
         case kFormSmallS: fa_small<D, kBf16, small_waves<D>(false)><<<grid, 64 * small_waves<D>(false), 0, s>>>(a); break;
-        default:
-            if constexpr (D == 64) {
-                if (p.form == kFormKeys8) fa_mfma_keys<64, 8, 1, kBf16><<<grid, 512, 0, s>>>(a);
-                else fa_mfma<64, 4, 1, kBf16><<<grid, 256, 0, s>>>(a);
-            }
+        case kFormKeys8:
+            if constexpr (D == 64) fa_mfma_keys<64, 8, 1, kBf16><<<grid, 512, 0, s>>>(a);
+            break;
+        default: fa_mfma<D, 4, 1, kBf16><<<grid, 256, 0, s>>>(a);
     }
     return launch_status();
 }
@@ -1557,7 +1575,8 @@ extern "C" int cdna3_attn_prefill_plan(const cdna3_prefill_cfg* cfg, int dtype, 
         out->rows = 16 * f32_tiles(c);
         out->grid = (long long)c.batch * c.nQHeads * ((c.seqQ + out->rows - 1) / out->rows);
     } else if (dtype == CDNA4_F16 || dtype == CDNA4_BF16) {
-        const PrefillPlan p = c.D == 128 ? plan_mfma<128>(c) : plan_mfma<64>(c);
+        const bool bf = dtype == CDNA4_BF16;
+        const PrefillPlan p = c.D == 128 ? plan_mfma<128>(c, bf) : plan_mfma<64>(c, bf);
         out->kernel = p.kernel;
         out->waves = p.waves;
         out->rows = p.rows;

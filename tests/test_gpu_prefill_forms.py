@@ -41,8 +41,18 @@ def test_keys_split_forms(D, SQ, SK, HQ, HK, B, causal, rows, dtype):
     _form(D, SQ, SK, HQ, HK, B, causal, dtype, rows, 8, heads, SQ + SK)
 
 
-def test_four_wave_form_d64():
-    _form(64, 301, 301, 32, 8, 6, 1, BF16, 64, 4, [(0, 0), (2, 9), (5, 31)], 3)
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("D,S,HQ,HK,B", [
+    (64, 301, 32, 8, 6),
+    (64, 65, 64, 64, 9),       # one query past a block, one key past a tile
+    (64, 129, 17, 17, 15),     # heads not a multiple of 8
+    (128, 144, 64, 16, 3),
+    (128, 65, 64, 64, 5),
+    (128, 129, 17, 17, 15),
+    (128, 316, 16, 4, 7),
+])
+def test_four_wave_form(D, S, HQ, HK, B, dtype):
+    _form(D, S, S, HQ, HK, B, 1, dtype, 64, 4, [(0, 0), (B // 2, HQ // 3), (B - 1, HQ - 1)], S + D)
 
 
 @pytest.mark.parametrize("D,S,HQ,HK,B,causal", [
