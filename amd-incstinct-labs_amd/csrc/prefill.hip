@@ -1320,8 +1320,8 @@ struct PrefillPlan { int kernel, waves, rows; long long grid; int form, order; }
 // Steps of q block i (heaviest last) and of a whole head, blocks of `rows` queries, `keys` per step
 // (one a multiple of the other).
 long long block_steps(const cdna3_prefill_cfg& c, int rows, int keys, long long i) {
-    const long long k = c.causal ? std::min<long long>(c.seqK, (i + 1) * rows) : c.seqK;
-    return (k + keys - 1) / keys;
+    const uint32_t k = (uint32_t)(c.causal ? std::min<long long>(c.seqK, (i + 1) * rows) : c.seqK);
+    return (k + (uint32_t)keys - 1u) / (uint32_t)keys;
 }
 double head_steps(const cdna3_prefill_cfg& c, int rows, int keys, long long nqb) {
     const double whole = (double)block_steps(c, rows, keys, nqb - 1);
@@ -1332,24 +1332,31 @@ double head_steps(const cdna3_prefill_cfg& c, int rows, int keys, long long nqb)
     return whole + (double)k * g * (g + 1) / 2 + (double)(n - k * g) * (g + 1);
 }
 
-// Largest load of a persistent workgroup (us) under an order of persistent_item.
-double pipe_load(const cdna3_prefill_cfg& c, const FormCost& fc, double step, int grid, int nqb, int nbh, int order) {
-    const int X = order ? 8 : 1, items = nbh * nqb;
-    double worst = 0.0;
-    for (int p = 0; p < grid; p += X) {   // the XCDs' lists are alike: XCD 0
-        double t = 0.0;
-        for (int item = p; item < items; item += grid) {
-            int bh, qrev;
-            persistent_item(item, grid, nqb, nbh, order, bh, qrev);
-            t += fc.fixed * (item == p ? 1.0 : fc.tail) + step * (double)block_steps(c, fc.rows, fc.keys, nqb - 1 - qrev);
-        }
-        worst = std::max(worst, t);
-    }
-    return worst;
-}
-
-constexpr long long kPipeSimItems = 1 << 15;       // larger grids: many rounds, taken as even
+constexpr int kPipeGroup = 512;    // workgroups of a group that pipe_load has room for
+constexpr int kPipeEntries = 1024;  // entries of a group's list that it walks: longer lists are taken as even
 constexpr double kPipeL2Bytes = 4.0 * 1024 * 1024; // an XCD's L2
+
+// Largest load of a persistent workgroup (us) under an order of persistent_item: one pass over the
+// item list of a group (the XCDs' lists are alike). At most kPipeEntries entries, because this runs
+// on the host ahead of every launch: a whole plan takes 2.4 us at B4 H32 S 8,192 (8.0 with a division
+// per item), 6.5 at most, 0.9 where nothing is walked; walks of up to 32,768 items took 45-210.
+double pipe_load(const cdna3_prefill_cfg& c, const FormCost& fc, double step, int grid, int nqb, int nbh, int order) {
+    const int sh = order ? 3 : 0, G = grid >> sh, H = nbh >> sh, list = H * nqb;
+    double load[kPipeGroup];
+    int qrev = 0, in_q = 0;   // of the entry, as persistent_item has them
+    for (int r0 = 0, r = 0; r0 < list; r0 += G, ++r) {
+        const int K = std::min(G, list - r0);
+        for (int j = 0; j < K; ++j) {
+            const int sp = (r & 1) ? K - 1 - j : j;
+            const double t = step * (double)block_steps(c, fc.rows, fc.keys, nqb - 1 - qrev);
+            if (r == 0) load[sp] = fc.fixed + t;
+            else load[sp] += fc.fixed * fc.tail + t;
+            if (order == 1) qrev = qrev + 1 == nqb ? 0 : qrev + 1;
+            else if (++in_q == H) { in_q = 0; ++qrev; }
+        }
+    }
+    return *std::max_element(load, load + std::min(G, list));
+}
 
 template <int D>
 PrefillPlan plan_mfma(const cdna3_prefill_cfg& c, bool bf16) {
@@ -1358,7 +1365,7 @@ PrefillPlan plan_mfma(const cdna3_prefill_cfg& c, bool bf16) {
     const long long blocks8 = heads * ((c.seqQ + 255) / 256);
     PrefillPlan best{};
     double best_t = 1e300;
-    for (int f = 0; f < kForms; ++f) {
+    for (int f = kForms - 1; f >= 0; --f) {   // fa_pipe last: its loads are added up only if they decide
         if (f == kFormKeys8 && D != 64) continue;
         // fa_mfma rounds its weights against one maximum per 64 keys where fa_small has one per wave and 32
         // keys, and lies 2-4 % further from 64 bits in fp16 (fa_pipe lies as far): it serves causal problems
@@ -1392,15 +1399,22 @@ PrefillPlan plan_mfma(const cdna3_prefill_cfg& c, bool bf16) {
             const int pcus = cus & ~7;
             if (pcus >= 8 && p.grid > pcus) p.grid = pcus;
             p.order = heads % 8 == 0 && p.grid % 8 == 0 ? 1 : 0;
-            t = std::max(fc.fixed + step * heavy, (fc.tail * fc.fixed * items + step * steps) / p.grid);
-            if (items > p.grid && items <= kPipeSimItems) {
+            const double even = std::max(fc.fixed + step * heavy, (fc.tail * fc.fixed * items + step * steps) / p.grid);
+            t = even;
+            const int group = (int)p.grid >> (p.order ? 3 : 0);
+            if (items > p.grid && !c.causal) {   // every block has the same steps: rounds of the fullest
+                const double rounds = (double)((items + p.grid - 1) / p.grid);
+                t = fc.fixed * (1.0 + fc.tail * (rounds - 1.0)) + step * heavy * rounds;
+            } else if (items > p.grid && even < best_t && group <= kPipeGroup &&
+                       items <= (long long)kPipeEntries * (p.order ? 8 : 1)) {
                 t = pipe_load(c, fc, step, (int)p.grid, (int)nqb, (int)heads, p.order);
-                if (p.order == 1 && c.causal) {
-                    // order 2 costs K/V sharing once an XCD's heads outgrow its L2 (B4 H32 S 8,192 1,683 ->
-                    // 1,825 us at equal balance; B2 40/8 S 5,000 606 -> 510, B7 8/1 S 2,675 155 -> 117)
-                    const double kv = 4.0 * c.seqK * c.D * std::max(1.0, heads / 8.0 / (c.nQHeads / c.nKVHeads));
+                // order 2 costs K/V sharing once an XCD's heads outgrow its L2 (B4 H32 S 8,192 1,683 ->
+                // 1,825 us at equal balance; B2 40/8 S 5,000 606 -> 510, B7 8/1 S 2,675 155 -> 117)
+                const double kv = 4.0 * c.seqK * c.D * std::max(1.0, heads / 8.0 / (c.nQHeads / c.nKVHeads));
+                const double cost2 = kv > kPipeL2Bytes ? 1.08 : 1.03;
+                if (p.order == 1 && even * cost2 < t) {
                     const double t2 = pipe_load(c, fc, step, (int)p.grid, (int)nqb, (int)heads, 2);
-                    if (t2 * (kv > kPipeL2Bytes ? 1.08 : 1.03) < t) {
+                    if (t2 * cost2 < t) {
                         t = t2;
                         p.order = 2;
                     }

@@ -1,5 +1,8 @@
 """The 16-bit prefill's choice of kernel (plan_mfma, csrc/prefill.hip), asked through the plan query on
 the CPU, where it plans for 256 CUs."""
+import ctypes
+import time
+
 import pytest
 
 import cdna4
@@ -15,3 +18,26 @@ def test_many_short_causal_sequences_take_four_waves_at_d128(c):
     # measured (us): the key-split forms 18.3, 23.4, 22.4, 22.2, fa_mfma 11.8, 19.9, 16.2, 16.6
     for dt in (cdna4.F16, cdna4.BF16):
         assert (plan(*c, dt).rows, plan(*c, dt).waves) == (64, 4)
+
+
+def test_planning_costs_little_at_every_size():
+    # Every call plans, so no shape may cost many times a small one's microsecond (a walk over all
+    # items had taken 45-200 us at the sizes below).
+    l, info = cdna4.lib(), cdna4.PlanInfo()
+
+    def cost(c):
+        cfg = cdna4.PrefillCfg(*c)
+        args = (ctypes.byref(cfg), cdna4.BF16, ctypes.byref(info))
+        best = 1e9
+        for _ in range(20):
+            t = time.perf_counter()
+            for _ in range(20):
+                l.cdna3_attn_prefill_plan(*args)
+            best = min(best, (time.perf_counter() - t) / 20)
+        return best
+
+    small = cost((64, 64, 64, 8, 8, 1, 1))
+    for c in [(128, 8192, 8192, 32, 32, 4, 1), (128, 2048, 2048, 32, 32, 100, 1), (128, 2048, 2048, 25, 25, 151, 1),
+              (64, 16, 16, 12, 12, 2000, 1), (64, 512, 512, 8, 8, 2000, 1), (128, 2048, 2048, 17, 17, 240, 1),
+              (128, 1700, 1700, 17, 17, 3, 1)]:
+        assert cost(c) < 8 * small, (c, cost(c), small)
