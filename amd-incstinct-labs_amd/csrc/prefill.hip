@@ -1392,6 +1392,8 @@ PrefillPlan plan_mfma(const cdna3_prefill_cfg& c, bool bf16) {
         p.rows = fc.rows;
         p.waves = f == kFormMfma4 ? 4 : (f == kFormSmallL || f == kFormSmallS) ? small_waves<D>(f == kFormSmallL) : 8;
         p.grid = items;
+        // a launch has fewer than 2^32 threads: beyond that only fa_pipe's persistent grid takes the items
+        if (f != kFormPipe && items * 64 * p.waves > 0xffffffffLL) continue;
         double t;
         if (f == kFormPipe) {
             // One resident workgroup per CU (LDS and VGPRs allow no second), so a grid of one workgroup

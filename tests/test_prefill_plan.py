@@ -12,6 +12,18 @@ def plan(D, SQ, SK, HQ, HK, B, causal, dtype=cdna4.BF16):
     return cdna4.prefill_plan(cdna4.PrefillCfg(D, SQ, SK, HQ, HK, B, causal), dtype)
 
 
+@pytest.mark.parametrize("c", [(64, 1, 1, 128, 128, 131072, 0), (128, 1, 1, 128, 128, 262144, 0),
+                               (64, 1, 1, 64, 64, 131071, 1), (64, 17, 17, 64, 64, 131072, 1),
+                               (128, 3, 70, 64, 8, 400000, 0), (64, 64, 64, 1, 1, 16777216, 1),
+                               (128, 129, 129, 8, 8, 2097152, 1)])
+def test_grids_fit_a_launch(c):
+    # fewer than 2^32 threads: what the one-workgroup-per-item forms cannot launch stays with the
+    # persistent grid
+    for dt in (cdna4.F16, cdna4.BF16):
+        p = plan(*c, dt)
+        assert p.grid * 64 * p.waves < 2 ** 32, (c, p.name, p.grid)
+
+
 @pytest.mark.parametrize("c", [(128, 144, 144, 64, 16, 3, 1), (128, 247, 247, 32, 32, 6, 1), (128, 165, 165, 6, 3, 42, 1),
                                (128, 316, 316, 16, 4, 7, 1)])
 def test_many_short_causal_sequences_take_four_waves_at_d128(c):
