@@ -107,7 +107,8 @@ class PlanInfo(ctypes.Structure):
 
 
 # CDNA4_KERNEL_* (include/cdna4_attn.h)
-KERNEL_NAMES = {1: "fa_mfma_8w", 2: "fa_mfma_4w", 3: "fa_small", 4: "fa_f32", 5: "decode_split", 6: "decode_wg"}
+KERNEL_NAMES = {1: "fa_mfma_8w", 2: "fa_mfma_4w", 3: "fa_small", 4: "fa_f32", 5: "decode_split", 6: "decode_wg",
+                7: "fa_mfma_keys"}
 
 
 def DecodeDmeCfg(D: int, N: int, nQHeads: int, nKVHeads: int, stride_kv: int, batch: int = 1) -> DecodeCfg:

@@ -1315,6 +1315,16 @@ constexpr FormCost form_cost(int f) {
     }
 }
 
+// The form's kernel as the plan query reports it.
+constexpr int form_kernel(int f) {
+    switch (f) {
+        case kFormPipe: return CDNA4_KERNEL_PREFILL_MFMA_8W;
+        case kFormMfma4: return CDNA4_KERNEL_PREFILL_MFMA_4W;
+        case kFormSmallL: case kFormSmallS: return CDNA4_KERNEL_PREFILL_SMALL;
+        default: return CDNA4_KERNEL_PREFILL_KEYS;
+    }
+}
+
 struct PrefillPlan { int kernel, waves, rows; long long grid; int form, order; };
 
 // Steps of q block i (heaviest last) and of a whole head, blocks of `rows` queries, `keys` per step
@@ -1389,6 +1399,7 @@ PrefillPlan plan_mfma(const cdna3_prefill_cfg& c, bool bf16) {
         const double step = fc.step * (1.0 + fc.load * util);
         PrefillPlan p{};
         p.form = f;
+        p.kernel = form_kernel(f);
         p.rows = fc.rows;
         p.waves = f == kFormMfma4 ? 4 : (f == kFormSmallL || f == kFormSmallS) ? small_waves<D>(f == kFormSmallL) : 8;
         p.grid = items;
@@ -1434,12 +1445,6 @@ PrefillPlan plan_mfma(const cdna3_prefill_cfg& c, bool bf16) {
             best = p;
         }
     }
-    // The reported kernel is the problem's size class (rows tells the form): whole rounds of 256-query
-    // blocks (a quarter of one when every block has the same work), 64-query blocks that fill the CUs
-    // twice, and the problems below that.
-    best.kernel = blocks8 >= (c.causal ? cus : cus / 4)              ? CDNA4_KERNEL_PREFILL_MFMA_8W
-                  : heads * ((c.seqQ + 63) / 64) >= 2LL * cus ? CDNA4_KERNEL_PREFILL_MFMA_4W
-                                                              : CDNA4_KERNEL_PREFILL_SMALL;
     return best;
 }
 

@@ -168,15 +168,14 @@ int cdna3_attn_decode_noalloc(const void* q, const void* K, const void* V, void*
  * CDNA4_ERR_INVALID_VALUE for arguments the entry point would reject.
  */
 enum {
-    /* 16-bit prefill: the size class of the problem; `rows` tells the form it takes (256: fa_pipe,
-       8 waves x 32 queries on a persistent grid; 128, 64, 32: 8 waves, the keys split over 2, 4 or 8
-       of them, or, with `waves` 4, fa_mfma; 16: fa_small, the keys split over its waves) */
-    CDNA4_KERNEL_PREFILL_MFMA_8W = 1,  /* 256-query blocks fill the CUs (non-causal: a quarter) */
-    CDNA4_KERNEL_PREFILL_MFMA_4W = 2,  /* 64-query blocks fill the CUs twice */
-    CDNA4_KERNEL_PREFILL_SMALL = 3,    /* anything below */
+    CDNA4_KERNEL_PREFILL_MFMA_8W = 1,  /* fa_pipe: 8 waves x 32 queries, persistent XCD-local grid */
+    CDNA4_KERNEL_PREFILL_MFMA_4W = 2,  /* fa_mfma: 4 waves x 16 queries, one workgroup per block */
+    CDNA4_KERNEL_PREFILL_SMALL = 3,    /* fa_small: 16 queries per workgroup, keys split over its waves */
     CDNA4_KERNEL_PREFILL_F32 = 4,      /* fa_f32: fp32 matrix-core kernel */
     CDNA4_KERNEL_DECODE_SPLIT = 5,     /* decode_mfma split-K grid + decode_merge */
-    CDNA4_KERNEL_DECODE_WG = 6         /* decode_wg: one launch, no workspace */
+    CDNA4_KERNEL_DECODE_WG = 6,        /* decode_wg: one launch, no workspace */
+    CDNA4_KERNEL_PREFILL_KEYS = 7      /* fa_mfma_keys: 8 waves, `rows` 128, 64 or 32 queries with the keys
+                                          split over 2, 4 or 8 groups of waves */
 };
 
 typedef struct {

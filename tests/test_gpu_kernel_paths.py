@@ -70,8 +70,7 @@ def check_prefill(D, SQ, SK, HQ, HK, B, causal, dtype, kernel, seed=0, heads=Non
     check_parity([o[b, h, rows] for b, h in heads], [want[(b, h)] for b, h in heads], dtype)
 
 
-# ---- fa_pipe<D, 8, 2> (plan name fa_mfma_8w): batch * heads * ceil(seqQ / 256) >= CUs (causal) --
-# ---- or >= CUs / 4 (non-causal) ---------------------------------------------------------------
+# ---- fa_pipe<D, 8, 2> (plan name fa_mfma_8w) ----------------------------------------------------
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_fa_mfma_8w_d128_causal_mha(dtype):
@@ -116,13 +115,14 @@ def test_fa_pipe_partial_odd_round():
                   heads=[(0, 0), (1, 9), (2, 18), (3, 31)])
 
 
-@pytest.mark.parametrize("D,S,H,dtype", [(128, 3000, 32, torch.bfloat16), (128, 2053, 32, torch.float16),
-                                         (64, 2085, 64, torch.float16)])
-def test_fa_pipe_causal_ragged_lengths(D, S, H, dtype):
+@pytest.mark.parametrize("D,S,H,dtype,kernel", [(128, 3000, 32, torch.bfloat16, "fa_mfma_8w"),
+                                                (128, 2053, 32, torch.float16, "fa_mfma_keys"),
+                                                (64, 2085, 64, torch.float16, "fa_mfma_8w")])
+def test_causal_ragged_lengths(D, S, H, dtype, kernel):
     # Causal (seqQ == seqK) at lengths that are not multiples of 32: the tail's fixed mask of the
     # chunk at a wave's first query and the general mask of the ragged last chunk apply to the
     # same chunk in some waves and to different chunks in others.
-    check_prefill(D, S, S, H, H, 1, 1, dtype, "fa_mfma_8w", seed=30 + S,
+    check_prefill(D, S, S, H, H, 1, 1, dtype, kernel, seed=30 + S,
                   heads=[(0, 0), (0, H // 2 - 1), (0, H - 1)])
 
 
@@ -133,52 +133,46 @@ def test_fa_pipe_short_keys(SK):
                   heads=[(0, 0), (0, 13), (0, 31)])
 
 
-# ---- fa_mfma<D, 4, 1>: mid-size problems --------------------------------------------------------
+# ---- fa_mfma_keys: mid-size problems (the form: test_gpu_prefill_forms.py) -----------------------
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_fa_mfma_4w_d128_causal(dtype):
-    check_prefill(128, 4096, 4096, 8, 8, 1, 1, dtype, "fa_mfma_4w", seed=7)
-
-
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_fa_mfma_4w_d64_gqa_causal(dtype):
-    check_prefill(64, 2048, 2048, 16, 4, 1, 1, dtype, "fa_mfma_4w", seed=8)
+def test_fa_mfma_keys_d128_causal(dtype):
+    check_prefill(128, 4096, 4096, 8, 8, 1, 1, dtype, "fa_mfma_keys", seed=7)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_fa_pipe_mid_size_d64_gqa_noncausal(dtype):
-    # 16 heads x 8 blocks of 256 queries = 128 < one round: the non-causal 8-wave plan with a grid of
-    # 128 workgroups, one work item each.
-    check_prefill(64, 2048, 2048, 16, 4, 1, 0, dtype, "fa_mfma_8w", seed=8)
+def test_fa_mfma_keys_d64_gqa_causal(dtype):
+    check_prefill(64, 2048, 2048, 16, 4, 1, 1, dtype, "fa_mfma_keys", seed=8)
 
 
-def test_fa_mfma_4w_ragged_causal():
-    check_prefill(128, 4093, 4093, 8, 2, 1, 1, torch.float16, "fa_mfma_4w", seed=9)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fa_mfma_keys_d64_gqa_noncausal(dtype):
+    check_prefill(64, 2048, 2048, 16, 4, 1, 0, dtype, "fa_mfma_keys", seed=8)
 
 
-def test_fa_pipe_mid_size_cross_attention():
-    # non-causal, seqK 1003 (ragged last tile), 8 x 16 = 128 blocks
-    check_prefill(64, 4096, 1003, 8, 8, 1, 0, torch.bfloat16, "fa_mfma_8w", seed=10)
+def test_fa_mfma_keys_ragged_causal():
+    check_prefill(128, 4093, 4093, 8, 2, 1, 1, torch.float16, "fa_mfma_keys", seed=9)
 
 
-def test_fa_pipe_quarter_round_noncausal():
-    # the smallest non-causal 8-wave plan: 64 blocks (one per XCD-aligned group), D 128
-    check_prefill(128, 2048, 2048, 8, 8, 1, 0, torch.bfloat16, "fa_mfma_8w", seed=13)
+def test_fa_mfma_keys_cross_attention():
+    # non-causal, seqK 1003 (ragged last step)
+    check_prefill(64, 4096, 1003, 8, 8, 1, 0, torch.bfloat16, "fa_mfma_keys", seed=10)
 
 
-# ---- fa_small: both workgroup forms -------------------------------------------------------------
+def test_fa_mfma_keys_noncausal_d128():
+    check_prefill(128, 2048, 2048, 8, 8, 1, 0, torch.bfloat16, "fa_mfma_keys", seed=13)
 
-@pytest.mark.parametrize("D,SQ,HQ,HK,B", [(128, 512, 8, 8, 1), (64, 700, 12, 4, 2)])
-def test_fa_small_forms(D, SQ, HQ, HK, B):
-    cfg = cdna4.PrefillCfg(D, SQ, SQ, HQ, HK, B, 1)
-    waves = cdna4.prefill_plan(cfg, torch.float16).waves
-    print(f"fa_small waves {waves}", flush=True)
-    check_prefill(D, SQ, SQ, HQ, HK, B, 1, torch.float16, "fa_small", seed=11)
+
+# ---- fa_small and its neighbour -----------------------------------------------------------------
+
+@pytest.mark.parametrize("D,SQ,HQ,HK,B,kernel", [(128, 512, 8, 8, 1, "fa_small"), (64, 700, 12, 4, 2, "fa_mfma_keys")])
+def test_small_causal_problems(D, SQ, HQ, HK, B, kernel):
+    check_prefill(D, SQ, SQ, HQ, HK, B, 1, torch.float16, kernel, seed=11)
 
 
 # ---- the strided entry point (the runtime's prompt path) against the oracle ----------------------
 
-@pytest.mark.parametrize("D,S,HQ,HK,dtype,kernel", [(64, 2048, 16, 4, torch.float16, "fa_mfma_4w"),
+@pytest.mark.parametrize("D,S,HQ,HK,dtype,kernel", [(64, 2048, 16, 4, torch.float16, "fa_mfma_keys"),
                                                      (128, 4096, 32, 8, torch.bfloat16, "fa_mfma_8w"),
                                                      (64, 300, 12, 12, torch.float16, "fa_small")])
 def test_prefill_strided_against_oracle(D, S, HQ, HK, dtype, kernel):
@@ -207,14 +201,13 @@ def test_prefill_strided_against_oracle(D, S, HQ, HK, dtype, kernel):
 
 
 def test_prefill_strided_rows_4gib_apart():
-    # K/V rows 2^25 elements apart: a 64-key tile spans 4 GiB, beyond the pipelined kernel's 32-bit
-    # per-lane copy offsets, so every tile takes the clamped copy with 64-bit addresses (the plan is
-    # still the 8-wave kernel). K and V share one ~4.5 GB allocation, heads interleaved in a row;
-    # only the rows used are written. seqK 70: one full and one partial tile.
+    # K/V rows 2^25 elements apart: a 64-key tile spans 4 GiB, beyond 32-bit per-lane copy offsets, so
+    # every step takes the clamped copy with 64-bit addresses. K and V share one ~4.5 GB allocation,
+    # heads interleaved in a row; only the rows used are written. seqK 70: one full and one partial tile.
     D, SQ, SK, HQ, HK = 128, 2048, 70, 8, 2
     rs = 1 << 25
     cfg = cdna4.PrefillCfg(D, SQ, SK, HQ, HK, 1, 0)
-    assert cdna4.prefill_plan(cfg, torch.bfloat16).name == "fa_mfma_8w"
+    assert cdna4.prefill_plan(cfg, torch.bfloat16).name == "fa_mfma_keys"
     g = torch.Generator(device=DEV).manual_seed(77)
     Q = _randn((HQ, SQ, D), torch.bfloat16, g)
     Kd = _randn((HK, SK, D), torch.bfloat16, g)

@@ -15,9 +15,11 @@ F16, BF16 = torch.float16, torch.bfloat16
 
 def _form(D, SQ, SK, HQ, HK, B, causal, dtype, rows, waves, heads, seed):
     p = cdna4.prefill_plan(cdna4.PrefillCfg(D, SQ, SK, HQ, HK, B, causal), dtype)
+    name = p.name
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert (p.rows, p.waves) == (rows, waves)
-    check_prefill(D, SQ, SK, HQ, HK, B, causal, dtype, p.name, seed=seed, heads=heads)
+        name = {256: "fa_mfma_8w", 16: "fa_small"}.get(rows, "fa_mfma_4w" if waves == 4 else "fa_mfma_keys")
+    check_prefill(D, SQ, SK, HQ, HK, B, causal, dtype, name, seed=seed, heads=heads)
 
 
 @pytest.mark.parametrize("dtype", [F16, BF16])

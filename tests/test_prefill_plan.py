@@ -1,15 +1,52 @@
 """The 16-bit prefill's choice of kernel (plan_mfma, csrc/prefill.hip), asked through the plan query on
-the CPU, where it plans for 256 CUs."""
+the CPU, where it plans for 256 CUs: what it reports is a form that exists, every grid fits a launch,
+and asking costs little, since every call asks."""
 import ctypes
+import math
+import random
 import time
 
 import pytest
 
 import cdna4
 
+# (kernel, waves, rows) of every form, by head dimension
+FORMS = {
+    64: {("fa_mfma_8w", 8, 256), ("fa_mfma_keys", 8, 128), ("fa_mfma_keys", 8, 64), ("fa_mfma_keys", 8, 32),
+         ("fa_mfma_4w", 4, 64), ("fa_small", 8, 16), ("fa_small", 4, 16)},
+    128: {("fa_mfma_8w", 8, 256), ("fa_mfma_keys", 8, 128), ("fa_mfma_keys", 8, 64), ("fa_mfma_4w", 4, 64),
+          ("fa_small", 4, 16), ("fa_small", 2, 16)},
+}
+
 
 def plan(D, SQ, SK, HQ, HK, B, causal, dtype=cdna4.BF16):
     return cdna4.prefill_plan(cdna4.PrefillCfg(D, SQ, SK, HQ, HK, B, causal), dtype)
+
+
+def shapes(count, seed):
+    rng = random.Random(seed)
+
+    def log_int(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    for _ in range(count):
+        causal = rng.choice([0, 1])
+        SQ = log_int(1, 9000)
+        HK = rng.choice([1, 2, 3, 8, 12, 17, 32])
+        yield (rng.choice([64, 128]), SQ, SQ if causal else log_int(1, 9000), HK * rng.choice([1, 2, 4, 8]), HK,
+               log_int(1, 200), causal), rng.choice([cdna4.F16, cdna4.BF16])
+
+
+def test_the_reported_kernel_is_the_form_that_runs():
+    seen = {64: set(), 128: set()}
+    for c, dt in shapes(6000, 1):
+        p = plan(*c, dt)
+        form = (p.name, p.waves, p.rows)
+        assert form in FORMS[c[0]], (c, form)
+        items = c[5] * c[3] * -(-c[1] // p.rows)
+        assert p.grid == (min(items, 256) if p.rows == 256 else items), (c, form, p.grid)
+        seen[c[0]].add(form)
+    assert seen == FORMS   # and every form is chosen somewhere
 
 
 @pytest.mark.parametrize("c", [(64, 1, 1, 128, 128, 131072, 0), (128, 1, 1, 128, 128, 262144, 0),
