@@ -24,6 +24,10 @@ pytestmark = pytest.mark.gpu
 _POOL = ThreadPoolExecutor(max_workers=8)   # the oracle is C called through ctypes (GIL released)
 
 
+def _cus():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
 def _randn(shape, dtype, g):
     return torch.randn(*shape, device=DEV, generator=g).to(dtype)
 
@@ -117,6 +121,7 @@ def test_fa_pipe_partial_odd_round():
 
 @pytest.mark.parametrize("D,S,H,dtype,kernel", [(128, 3000, 32, torch.bfloat16, "fa_mfma_8w"),
                                                 (128, 2053, 32, torch.float16, "fa_mfma_keys"),
+                                                (128, 2053, 64, torch.float16, "fa_mfma_8w"),
                                                 (64, 2085, 64, torch.float16, "fa_mfma_8w")])
 def test_causal_ragged_lengths(D, S, H, dtype, kernel):
     # Causal (seqQ == seqK) at lengths that are not multiples of 32: the tail's fixed mask of the
@@ -131,6 +136,18 @@ def test_fa_pipe_short_keys(SK):
     # Fewer keys than the pipelined main loop needs (t_main = 0 below 96): every tile in the tail.
     check_prefill(128, 4096, SK, 32, 32, 1, 0, torch.float16, "fa_mfma_8w", seed=12 + SK,
                   heads=[(0, 0), (0, 13), (0, 31)])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D,SQ,SK,HQ,HK,B", [
+    (64, 2048, 2048, 16, 4, 2),    # one round of 256 workgroups, grouped-query heads
+    (64, 4096, 1003, 8, 8, 2),     # cross attention, a ragged last tile
+    (64, 1325, 1068, 8, 2, 5),     # fewer items than CUs
+    (128, 1100, 270, 16, 2, 2),
+])
+def test_fa_pipe_one_round_noncausal(D, SQ, SK, HQ, HK, B, dtype):
+    check_prefill(D, SQ, SK, HQ, HK, B, 0, dtype, "fa_mfma_8w", seed=SQ + SK,
+                  heads=[(0, 0), (0, HQ - 1), (B - 1, HQ // 2)])
 
 
 # ---- fa_mfma_keys: mid-size problems (the form: test_gpu_prefill_forms.py) -----------------------
@@ -163,17 +180,37 @@ def test_fa_mfma_keys_noncausal_d128():
     check_prefill(128, 2048, 2048, 8, 8, 1, 0, torch.bfloat16, "fa_mfma_keys", seed=13)
 
 
-# ---- fa_small and its neighbour -----------------------------------------------------------------
+# ---- fa_small: both workgroup forms, and its neighbour ------------------------------------------
 
 @pytest.mark.parametrize("D,SQ,HQ,HK,B,kernel", [(128, 512, 8, 8, 1, "fa_small"), (64, 700, 12, 4, 2, "fa_mfma_keys")])
 def test_small_causal_problems(D, SQ, HQ, HK, B, kernel):
     check_prefill(D, SQ, SQ, HQ, HK, B, 1, torch.float16, kernel, seed=11)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D,SQ,SK,HQ,HK,B,causal,waves", [
+    # one round of workgroups: all of a CU's LDS
+    (64, 300, 300, 12, 12, 1, 1, 8), (64, 1000, 830, 4, 2, 1, 0, 8), (64, 17, 33, 3, 1, 2, 0, 8),
+    (128, 249, 249, 12, 12, 1, 1, 4), (128, 40, 206, 8, 8, 5, 0, 4),
+    # more: two workgroups per CU, half as many waves each
+    (64, 239, 239, 17, 17, 2, 1, 4), (64, 113, 113, 17, 17, 2, 1, 4), (64, 94, 60, 17, 17, 5, 0, 4),
+    (64, 5, 1155, 34, 17, 14, 0, 4),
+    (128, 100, 100, 32, 32, 2, 1, 2), (128, 77, 77, 32, 8, 3, 1, 2), (128, 99, 131, 8, 8, 5, 0, 2),
+    (128, 1, 220, 64, 32, 11, 0, 2),
+])
+def test_fa_small_forms(D, SQ, SK, HQ, HK, B, causal, waves, dtype):
+    if _cus() == 256:
+        p = cdna4.prefill_plan(cdna4.PrefillCfg(D, SQ, SK, HQ, HK, B, causal), dtype)
+        assert (p.name, p.rows, p.waves) == ("fa_small", 16, waves)
+    check_prefill(D, SQ, SK, HQ, HK, B, causal, dtype, "fa_small", seed=SQ + SK + B)
+
+
 # ---- the strided entry point (the runtime's prompt path) against the oracle ----------------------
 
 @pytest.mark.parametrize("D,S,HQ,HK,dtype,kernel", [(64, 2048, 16, 4, torch.float16, "fa_mfma_keys"),
                                                      (128, 4096, 32, 8, torch.bfloat16, "fa_mfma_8w"),
+                                                     (64, 300, 64, 16, torch.float16, "fa_mfma_4w"),
+                                                     (128, 541, 64, 16, torch.bfloat16, "fa_mfma_4w"),
                                                      (64, 300, 12, 12, torch.float16, "fa_small")])
 def test_prefill_strided_against_oracle(D, S, HQ, HK, dtype, kernel):
     max_seq = (S + 100 + 7) // 8 * 8
@@ -200,14 +237,26 @@ def test_prefill_strided_against_oracle(D, S, HQ, HK, dtype, kernel):
     check_parity([o[rows, h] for _, h in heads], [want[(0, h)] for _, h in heads], dtype)
 
 
-def test_prefill_strided_rows_4gib_apart():
-    # K/V rows 2^25 elements apart: a 64-key tile spans 4 GiB, beyond 32-bit per-lane copy offsets, so
-    # every step takes the clamped copy with 64-bit addresses. K and V share one ~4.5 GB allocation,
-    # heads interleaved in a row; only the rows used are written. seqK 70: one full and one partial tile.
-    D, SQ, SK, HQ, HK = 128, 2048, 70, 8, 2
-    rs = 1 << 25
-    cfg = cdna4.PrefillCfg(D, SQ, SK, HQ, HK, 1, 0)
-    assert cdna4.prefill_plan(cfg, torch.bfloat16).name == "fa_mfma_keys"
+@pytest.mark.parametrize("D,SQ,SK,HQ,HK,causal,rs,rows", [
+    # 2^25 elements: a 64-key tile spans 4 GiB, beyond 32-bit per-lane copy offsets, in every form; seqK 70 is
+    # one full and one partial tile
+    (128, 4096, 70, 32, 2, 0, 1 << 25, 256),
+    (128, 2048, 70, 8, 2, 0, 1 << 25, 64),
+    (64, 64, 70, 8, 2, 0, 1 << 25, 16),
+    (64, 300, 300, 64, 16, 1, 1 << 25, 64),
+    (128, 1600, 300, 16, 2, 0, 1 << 25, 128),
+    # a 64-key tile still fits, the 128- and 256-key steps of fa_mfma_keys do not
+    (128, 800, 400, 8, 8, 0, (1 << 24) + (1 << 18), 64),
+    (64, 2328, 900, 3, 3, 0, (1 << 23) + (1 << 16), 32),
+])
+def test_prefill_strided_rows_far_apart(D, SQ, SK, HQ, HK, causal, rs, rows):
+    # Every step then takes the clamped copy with 64-bit addresses. K and V share one allocation (up to
+    # 20 GB), heads interleaved in a row; only the rows used are written.
+    cfg = cdna4.PrefillCfg(D, SQ, SK, HQ, HK, 1, causal)
+    plan = cdna4.prefill_plan(cfg, torch.bfloat16)
+    print(f"rows {rs} elements apart -> {plan.name} rows {plan.rows}", flush=True)
+    if _cus() == 256:
+        assert plan.rows == rows
     g = torch.Generator(device=DEV).manual_seed(77)
     Q = _randn((HQ, SQ, D), torch.bfloat16, g)
     Kd = _randn((HK, SK, D), torch.bfloat16, g)
@@ -220,16 +269,16 @@ def test_prefill_strided_rows_4gib_apart():
     cdna4.prefill_strided(Q, big, big[HK * D:], O, cfg, st)
     torch.cuda.synchronize()
     assert torch.isfinite(O.float()).all()
-    rows = _rows(SQ, 5)
+    check = _rows(SQ, 5)
     q = Q.float().cpu().numpy()[None]
     k = Kd.float().cpu().numpy()[None]
     v = Vd.float().cpu().numpy()[None]
-    heads = [(0, h) for h in range(HQ)]
-    want = _oracle_heads(q, k, v, heads, rows, D, SQ, SK, HQ, HK, 0)
+    heads = [(0, h) for h in range(0, HQ, max(1, HQ // 8))]
+    want = _oracle_heads(q, k, v, heads, check, D, SQ, SK, HQ, HK, causal)
     o = O.float().cpu().numpy()
     del big
     torch.cuda.empty_cache()
-    check_parity([o[h, rows] for _, h in heads], [want[(0, h)] for _, h in heads], torch.bfloat16)
+    check_parity([o[h, check] for _, h in heads], [want[(0, h)] for _, h in heads], torch.bfloat16)
 
 
 # ---- BASELINE config 3 at full size: every head of batches 0 and 3 -------------------------------
@@ -318,10 +367,6 @@ def test_decode_split_more_than_64_partials():
     # batch 1 with one kv head: P > 64, so the merge runs several 64-partial passes.
     plan = check_decode(128, 65536, 4, 1, 1, torch.float16, "decode_split", seed=3)
     assert plan.partials > 64
-
-
-def _cus():
-    return torch.cuda.get_device_properties(0).multi_processor_count
 
 
 def test_decode_whole_rounds_one_launch_d64_streaming():
