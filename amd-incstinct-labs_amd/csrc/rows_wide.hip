@@ -72,13 +72,36 @@ __device__ __forceinline__ f32x4 own(f32x4 v, int sk, float mean = 0.f) {
     for (int e = 0; e < 4; ++e) v[e] = e >= sk ? v[e] - mean : 0.f;
     return v;
 }
-// Sums of a vector, in pairs as in the wave-per-row kernels, whose results unaligned rows of one wave then
-// give bit for bit. Error against 64 bits, softmax: in sequence 6.5e-8 at 2,047 columns, 5.9e-8 at 5,000,
-// in pairs 5.6e-8 and 5.4e-8 (element-wise kernels 6.1e-8, 7.4e-8). Rows a little wider than 64 or 128
-// keep 2-6 % more than the element-wise kernels (67: 6.4e-8 -> 6.7e-8): their last vector is alone in
-// its 16 lanes, one more addition at the row's full size.
-__device__ __forceinline__ float sum4(f32x4 v) { return (v[0] + v[1]) + (v[2] + v[3]); }
-__device__ __forceinline__ float sumsq4(f32x4 v) { return (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); }
+// A vector added to a thread's sum. Rows of one wave add its elements in pairs, as the wave-per-row
+// kernels do, whose results unaligned rows then give bit for bit: in sequence they were further from 64
+// bits than the element-wise kernels (softmax of 2,047 columns 6.5e-8 relative, in pairs 5.6e-8,
+// element-wise 6.1e-8; a little above 64 or 128 columns 2-6 % over those remain, 67: 6.4e-8 -> 6.7e-8: the
+// last vector is alone in its 16 lanes, one more addition at the row's full size). Rows of a workgroup
+// have short sums per thread and add in sequence (32,000 columns: 4.9e-8, in pairs 5.0e-8, element-wise
+// 6.4e-8).
+template <int TPR>
+__device__ __forceinline__ void add4(float& s, f32x4 v, int sk) {
+    if constexpr (TPR == 64) {
+        v = own(v, sk);
+        s += (v[0] + v[1]) + (v[2] + v[3]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += e >= sk ? v[e] : 0.f;
+    }
+}
+template <int TPR>
+__device__ __forceinline__ void add4_squares(float& s, f32x4 v, int sk, float mean) {
+    if constexpr (TPR == 64) {
+        v = own(v, sk, mean);
+        s += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float d = v[e] - mean;
+            s += e >= sk ? d * d : 0.f;
+        }
+    }
+}
 
 constexpr int kBlock = 256;
 
@@ -113,7 +136,7 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rows_kernel(const
         for (int k = 0; k < NV; ++k) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[k][e] = __expf(v[k][e] - m);
-            s += sum4(own(v[k], skip(k)));
+            add4<TPR>(s, v[k], skip(k));
         }
         const float inv = 1.f / row_combine<TPR>(s, Sum{}, slots[1]);
 #pragma unroll
@@ -126,13 +149,12 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rows_kernel(const
         if constexpr (kOp == kRowsLayer) {
             float s = 0.f;
 #pragma unroll
-            for (int k = 0; k < NV; ++k) s += sum4(own(v[k], skip(k)));
+            for (int k = 0; k < NV; ++k) add4<TPR>(s, v[k], skip(k));
             mean = row_combine<TPR>(s, Sum{}, slots[0]) / (float)H;
         }
         float q = 0.f;
 #pragma unroll
-        for (int k = 0; k < NV; ++k)
-            q += sumsq4(own(v[k], skip(k), mean));
+        for (int k = 0; k < NV; ++k) add4_squares<TPR>(q, v[k], skip(k), mean);
         const float inv = rsqrtf(row_combine<TPR>(q, Sum{}, slots[1]) / (float)H + eps);
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
