@@ -518,8 +518,8 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows(const uint16_t* __r
 }
 
 // Shapes gemm_rows takes: one round of workgroups (8192 x 2048 at M 1 and 16: ring 9.7 and 9.8 us, here
-// 10.0 and 12.6) and a K of four stages (1024 x 256: 2.8 -> 2.3, 2.9 -> 2.5); the tile query's callers
-// rely on the ring below that.
+// 10.0 and 12.6) and a K of four stages (1024 x 256: 2.8 -> 2.3, 2.9 -> 2.5). Below that the ring is kept
+// and not measured against: the tile query's tests hold its tiles there.
 bool takes_rows(int M, int ncols, int K, int cus) {
     return M <= kRowsMax && K >= 4 * kBK && (ncols + 15) / 16 <= cus;
 }
@@ -589,8 +589,9 @@ constexpr double kStageUs = 0.1;           // per 64-wide K stage
 constexpr double kCuBytesPerUs = 2.0e5;    // ~200 GB/s of operand tiles per CU
 constexpr double kCuFlopsPerUs = 8.0e6;    // ~8 TFLOP/s of fp16 MFMA per CU
 
-// Plain products of fewer stages stay on the ring's menu, whose tiles the existing callers of the tile
-// query rely on there (4096 x 4096 x 256, fp32 out: ring 27.5 us, 256 x 256 21.7).
+// Plain products of fewer stages stay on the ring's menu: not a limit of the kernel (two stages do), and not
+// the faster side either (4096 x 4096 x 256, fp32 out: ring 27.5 us, 256 x 256 21.7), but the tiles
+// that the tile query's tests name for these shapes.
 constexpr int kBigMinStages = 5;
 
 Tile pick_tile(int M, int N, int K, int cus, bool silu = false) {
@@ -617,7 +618,7 @@ Tile pick_tile(int M, int N, int K, int cus, bool silu = false) {
 // round of one workgroup per CU, fitted to a sweep of both tiles and the ring over M 200 .. 4096 at
 // N x K of 768 x 768 .. 8192 x 4096 (14 pairs; fill: share of the CUs the tiles occupy, at most 1): a
 // tile's prologue and epilogue, then its stages. The estimate picked the faster side at each sweep
-// point beyond 4 %; small products stay on the ring (512 x 8192 x 4096: ring 45.9, 256 x 128 78.9).
+// point beyond 4 %, and no product of profiles/gemm_tiles.md is over 4 % slower than on the ring; small products stay on the ring (512 x 8192 x 4096: ring 45.9, 256 x 128 78.9).
 Tile pick_big(int M, int N, int K, int cus, bool silu, const Tile& t) {
     const int nk = K / kBK;
     if (nk < (silu ? 2 : kBigMinStages)) return Tile{0, 0};

@@ -73,6 +73,8 @@ constexpr size_t group_tile(size_t group, unsigned wave, int waves) { return gro
 // most one tile per CU, then 8 and 16 with up to two (262,144 f32: 256 tiles 4.1, 512 tiles 5.1;
 // 1,000,003 f32: 489 tiles of 8 vectors 6.9, 245 of 16 7.6). Against groups of large tiles:
 // 1,000 elements 6.1 -> 3.5, 11.8 -> 3.6, 8.2 -> 4.1; 1,000,003 12.4 -> 7.1, 18.2 -> 7.0, 18.8 -> 9.0.
+// No line by alignment: 16-bit inputs at elements 0 / 1 / 2 / 3 take 3.2 / 3.3 / 3.3 / 3.2 at 1,000, 6.7 /
+// 6.4 / 6.7 / 6.9 at 1,000,000 and, in small tiles, 8.6 / 9.0 / 8.8 / 8.9 at 3,000,000.
 constexpr int kSpreadTiles = 512;
 constexpr int kSpreadMaxU = 16;
 constexpr int spread_u(size_t n, int VEC) {

@@ -202,10 +202,10 @@ int cdna3_attn_decode_plan(const cdna3_decode_cfg* cfg, int dtype, int with_work
  * Workspace: >= the returned size. The scan's look-back flags carry a per-call epoch, so a
  * workspace needs no clearing between calls (one launch per call, plus a one-wave tail launch
  * for the last n % 4 elements of a large aligned call). A captured call also clears its flags, so
- * that every replay of the graph waits for its own. A zeroed workspace, or one last used by
- * another scan, is always safe; memory never written by a scan is accepted too, with the caveat
- * that a 64-bit word of it whose upper half happens to equal the call's 32-bit tag would be read
- * as published (so zero a fresh workspace once to rule that out).
+ * that every replay of the graph waits for its own. A zeroed workspace is always safe. Other memory
+ * (never written by a scan, or last used by a scan of another size, whose tile totals may lie where
+ * this call's flags do) is accepted too, with the caveat that a 64-bit word of it whose upper half
+ * happens to equal the call's 32-bit tag would be read as published.
  * Scan status: the scan's decoupled look-back waits a bounded time for a predecessor tile; if a
  * wait ever exceeds that bound the result is not valid and the call marks the workspace
  * (its first word takes the call's epoch, the second word holds the epoch of the latest call).
@@ -238,6 +238,8 @@ int cdna3_softmax_rows_f32(const float* X, float* Y, int M, int H, cdna4_stream_
  * cdna3_layernorm_f32 replaces the two-pass DPP layernorm_kernel (research/
  * wave-primitives/benchmarks/bench_layernorm.hip:51-114) with runtime H:
  * Y = (X - mean) * rsqrt(var + eps) * gamma + beta, var = mean((X - mean)^2).
+ * Sums of a row are fp32; their order, and so the last bits, depends on M for 768 columns and more
+ * (up to 512 or 1,024 rows a workgroup adds a row, above that a wave), for the row softmax as well.
  * cdna3_rope_f16 replaces rope_kernel (forward.hpp:135-148): rotate-half RoPE in place
  * on T fp16 [seq][heads][D] with cos/sin fp32 [seq][D]; each (d, d+D/2) pair is read
  * and written by one thread (the reference updates the pair from two threads).
@@ -261,7 +263,9 @@ int cdna3_rope_table_f32(float* cos_tab, float* sin_tab, int pos0, int T, int D,
  * (cdna3-prims/include/cdna3/runtime/rocblas_gemm.hpp:8-20, forward.hpp:70-131; beta 0 or 1).
  * Returns CDNA4_ERR_INVALID_VALUE, launching nothing, when K is not a multiple of 64, N or ldy
  * not a multiple of 4, ldy < N, X or W not 16-byte aligned or Y not 16- (fp32) or 8-byte (fp16)
- * aligned (the session then calls rocBLAS).
+ * aligned (the session then calls rocBLAS). Where the few-row kernel takes a product (M <= 16, K >= 256,
+ * N up to 16 columns per CU) K is added in eight parts, otherwise in one: a row's last bits then
+ * differ between M <= 16 and M > 16, and between no other M.
  */
 int cdna4_gemm_f16_nt(const void* X, const void* W, void* Y, int y_f32, int accum, int M, int N,
                       int K, int ldy, cdna4_stream_t stream);

@@ -55,7 +55,7 @@ def parity_err(got: np.ndarray, ref: np.ndarray, dtype: torch.dtype) -> float:
 
 def tolerance(dtype: torch.dtype) -> float:
     """Parity bound per output dtype for parity_err: 1e-4 (fp32), 2e-3 (fp16 and bf16), the
-    tolerances the north star states; bf16 additionally allows the output's own rounding (above)."""
+    project's tolerances; bf16 additionally allows the output's own rounding (above)."""
     return {torch.float32: 1e-4, torch.float16: 2e-3, torch.bfloat16: 2e-3}[dtype]
 
 

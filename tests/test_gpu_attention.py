@@ -42,7 +42,7 @@ def test_prefill_reference_validation_set(cfg, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_prefill_fa2_reference_config(dtype):
-    # B1 H8 S512 D64, non-causal, U(-1,1) fp32 from seed 42; fp16-rounded arm.
+    # The FA2 reference configuration: B1 H8 S512 D64, non-causal, U(-1,1) fp32 from seed 42; fp16-rounded arm.
     got, ref, _ = prefill_case(64, 512, 512, 8, 8, 1, 0, dtype, seed=42, dist="uniform")
     if dtype == torch.float32:
         check_abs(got, ref, 1e-4, what="cfg1 (B1 H8 S512 D64) fp32 arm, abs")
@@ -76,7 +76,7 @@ def test_prefill_closed_forms(dtype):
 
 
 def test_prefill_full_size_config_subsample():
-    # BASELINE config 3 shape (B4 H32 S8192 D128 causal bf16). Heads are independent, so the
+    # The large causal prefill (B4 H32 S8192 D128 causal bf16). Heads are independent, so the
     # oracle-generated heads below are checked inside otherwise random full-size tensors.
     B, H, S, D = 4, 32, 8192, 128
     torch.manual_seed(0)
@@ -145,7 +145,7 @@ def test_decode_strided_cache(dtype):
 
 
 def test_decode_full_size_config_and_split_invariance():
-    # batch 32, 32 q heads / 8 kv heads, D128, N8192, fp16 N(0,1).
+    # The batched decode: batch 32, 32 q heads / 8 kv heads, D128, N8192, fp16 N(0,1).
     B, HQ, HK, D, N = 32, 32, 8, 128, 8192
     torch.manual_seed(1)
     q = torch.randn(B, HQ, D, device=DEV, dtype=torch.float16)
@@ -181,7 +181,7 @@ def test_decode_full_size_config_and_split_invariance():
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_decode_full_size_config_on_the_split_k_plan(monkeypatch, dtype):
-    # BASELINE config 4 names split-K across workgroups with a DPP final reduce: the same shape on
+    # That configuration names split-K across workgroups with a DPP final reduce: the same shape on
     # that plan (forced; the one-launch plan is the default on a 256-CU part), against the oracle;
     # fp16 as the config, and bf16 at the same size.
     B, HQ, HK, D, N = 32, 32, 8, 128, 8192

@@ -281,7 +281,7 @@ def test_prefill_strided_rows_far_apart(D, SQ, SK, HQ, HK, causal, rs, rows):
     check_parity([o[h, check] for _, h in heads], [want[(0, h)] for _, h in heads], torch.bfloat16)
 
 
-# ---- BASELINE config 3 at full size: every head of batches 0 and 3 -------------------------------
+# ---- the large causal prefill (B4 H32 S8192 D128) at full size: every head of batches 0 and 3 -----
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_prefill_config3_subsample_every_head_of_batches_0_and_3(dtype):

@@ -223,7 +223,7 @@ def test_cfg5_shape_matches_oracle(tmp_path):
 
 
 def test_cfg5_full_workload_matches_oracle(tmp_path):
-    # BASELINE config 5 exactly as bench.py runs it (Session::generate, session.hpp:263-296): the
+    # The 12-layer decoder exactly as bench.py runs it (Session::generate, session.hpp:263-296): the
     # bench's model (seed 5), its 512-token prompt (default_rng(5)) and 128 greedy tokens. Every
     # step's logits against the oracle under teacher forcing (the oracle runs the prompt and the
     # 127 tokens the GPU fed back, ~20 s on one host thread), every token against the oracle's

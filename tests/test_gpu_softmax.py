@@ -4,7 +4,7 @@ Bound, element-wise: |gpu - ref| <= ref * (1e-6 + 1.2e-7 * |x - max|) + 1e-37. T
 computes exp(x - m) as 2^((x - m) * log2 e): rounding the product to fp32 moves the result by a
 relative 2^-24 * |x - m| * log2(e) * ln(2) = 6e-8 * |x - m| (the slope, doubled), the exponential
 itself by about one fp32 ulp, the row sum and the final product by a few more. The oracle takes
-exp and the sum in double. The same outputs are also held to the north star's fp32 tolerance
+exp and the sum in double. The same outputs are also held to the project's fp32 tolerance
 (1e-4, absolute below 1) for the run's parity table."""
 import ctypes
 
